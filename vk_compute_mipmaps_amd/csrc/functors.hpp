@@ -16,6 +16,8 @@
 //   store(t, v)          NVPRO_PYRAMID_STORE: Val -> Raw
 //   add, mul, reduce3    the arithmetic REDUCE, REDUCE2 and REDUCE4 are built
 //                        from (box, reduce2, reduce3 below)
+//   Acc, first3, next3,  reduce3 tap by tap: done3(next3(w2, v2, next3(w1, v1,
+//   done3                first3(w0, v0)))) is reduce3(w0, v0, w1, v1, w2, v2)
 //   kPrescale            whether load<true> then box<true> equals box<false>
 //                        of plain loads bit for bit (exact scaling by 0.25)
 //
@@ -77,6 +79,14 @@ struct Fp32Arith
   {
     return fma3(w0, v0, w1, v1, w2, v2);
   }
+  using Acc = float4;
+  __device__ static Acc first3(float w, Val v) { return f4mul(v, w); }
+  __device__ static Acc next3(float w, Val v, Acc a)
+  {
+    return make_float4(__builtin_fmaf(w, v.x, a.x), __builtin_fmaf(w, v.y, a.y), __builtin_fmaf(w, v.z, a.z),
+                       __builtin_fmaf(w, v.w, a.w));
+  }
+  __device__ static Val done3(Acc a) { return a; }
 };
 
 // NVPRO_PYRAMID_REDUCE2 of srgba8_mipmap_preamble.glsl:35: 0.5 * (v0 + v1).
@@ -143,12 +153,49 @@ struct Srgba8 : Fp32Arith
   static_assert(NVPRO_SRGB_ENC_BUCKETS % 4u == 0u, "16-byte table loads");
   static_assert(23u - NVPRO_SRGB_ENC_MANT_BITS == 16u, "the floats of a bucket differ in their low 16 bits");
 
+  // The fill in two halves, so that a kernel can issue its own loads between
+  // the table's and the wait for them.  No branches: a conditional load would
+  // end a block that the scheduler cannot cross.  Threads past the tables' end
+  // load and store words of other threads again, each its own (one word from
+  // many lanes would serialise the LDS write).
+  template <int BS>
+  struct TableLoads
+  {
+    static constexpr int kEnc = (NVPRO_SRGB_ENC_BUCKETS / 4 + BS - 1) / BS;
+    uint4 e[kEnc], d;
+  };
+  template <int BS>
+  __device__ static uint32_t encWord(int k)
+  {
+    constexpr uint32_t N = NVPRO_SRGB_ENC_BUCKETS / 4u, spare = TableLoads<BS>::kEnc * BS - N;
+    static_assert(spare <= N, "every thread has a word");
+    const uint32_t i = threadIdx.x + k * BS;
+    return i < N ? i : i - spare;
+  }
+  template <int BS>
+  __device__ static void fillLoad(TableLoads<BS>& r)
+  {
+#pragma unroll
+    for(int k = 0; k < TableLoads<BS>::kEnc; ++k)
+      r.e[k] = reinterpret_cast<const uint4*>(gSrgbEncode)[encWord<BS>(k)];
+    r.d = reinterpret_cast<const uint4*>(gSrgbDecode)[threadIdx.x & 63u];
+  }
+  template <int BS>
+  __device__ static void fillStore(Tables& t, const TableLoads<BS>& r, float scale)
+  {
+    reinterpret_cast<float4*>(t.dec)[threadIdx.x & 63u] =
+        make_float4(__uint_as_float(r.d.x) * scale, __uint_as_float(r.d.y) * scale, __uint_as_float(r.d.z) * scale,
+                    __uint_as_float(r.d.w) * scale);
+#pragma unroll
+    for(int k = 0; k < TableLoads<BS>::kEnc; ++k)
+      reinterpret_cast<uint4*>(t.enc)[encWord<BS>(k)] =
+          make_uint4(r.e[k].x ^ 0xffffu, r.e[k].y ^ 0xffffu, r.e[k].z ^ 0xffffu, r.e[k].w ^ 0xffffu);
+  }
   template <int BS>
   __device__ static void fill(Tables& t, float scale)
   {
     // 16-byte loads, every global load issued before any LDS store.
     constexpr int kEnc = (NVPRO_SRGB_ENC_BUCKETS / 4 + BS - 1) / BS;
-    static_assert(BS >= 64, "the decode table is one 16-byte load per thread of the first 64");
     const uint4* genc = reinterpret_cast<const uint4*>(gSrgbEncode);
     uint4 e[kEnc];
 #pragma unroll
@@ -167,8 +214,13 @@ struct Srgba8 : Fp32Arith
     {
       const uint32_t i = threadIdx.x + k * BS;
       if(i < NVPRO_SRGB_ENC_BUCKETS / 4u)
+      {
+        // Keeps the compiler from moving the complement up to each load, which
+        // would wait for every load before issuing the next.
+        __asm__ volatile("" : "+v"(e[k].x), "+v"(e[k].y), "+v"(e[k].z), "+v"(e[k].w));
         reinterpret_cast<uint4*>(t.enc)[i] =
             make_uint4(e[k].x ^ 0xffffu, e[k].y ^ 0xffffu, e[k].z ^ 0xffffu, e[k].w ^ 0xffffu);
+      }
     }
   }
 
@@ -254,6 +306,18 @@ struct Rgba32f : Fp32Arith
   };
   using DualTables = Tables;
   template <int BS>
+  struct TableLoads
+  {
+  };
+  template <int BS>
+  __device__ static void fillLoad(TableLoads<BS>&)
+  {
+  }
+  template <int BS>
+  __device__ static void fillStore(Tables&, const TableLoads<BS>&, float)
+  {
+  }
+  template <int BS>
   __device__ static void fill(Tables&, float)
   {
   }
@@ -288,6 +352,18 @@ struct Rgba16f : Fp32Arith
     int unused;
   };
   using DualTables = Tables;
+  template <int BS>
+  struct TableLoads
+  {
+  };
+  template <int BS>
+  __device__ static void fillLoad(TableLoads<BS>&)
+  {
+  }
+  template <int BS>
+  __device__ static void fillStore(Tables&, const TableLoads<BS>&, float)
+  {
+  }
   template <int BS>
   __device__ static void fill(Tables&, float)
   {
@@ -328,6 +404,18 @@ struct Rgba16fPacked
   using Tables     = Rgba16f::Tables;
   using DualTables = Tables;
   template <int BS>
+  struct TableLoads
+  {
+  };
+  template <int BS>
+  __device__ static void fillLoad(TableLoads<BS>&)
+  {
+  }
+  template <int BS>
+  __device__ static void fillStore(Tables&, const TableLoads<BS>&, float)
+  {
+  }
+  template <int BS>
   __device__ static void fill(Tables&, float)
   {
   }
@@ -350,6 +438,18 @@ struct Rgba16fPacked
   {
     const __half2 k = __float2half2_rn(s);  // 0.25 and 0.5 are exact in binary16
     return Val{__hmul2(a.rg, k), __hmul2(a.ba, k)};
+  }
+  using Acc = float4;
+  __device__ static float4 widen(Val v)
+  {
+    const float2 rg = __half22float2(v.rg), ba = __half22float2(v.ba);
+    return make_float4(rg.x, rg.y, ba.x, ba.y);
+  }
+  __device__ static Acc first3(float w, Val v) { return Fp32Arith::first3(w, widen(v)); }
+  __device__ static Acc next3(float w, Val v, Acc a) { return Fp32Arith::next3(w, widen(v), a); }
+  __device__ static Val done3(Acc a)
+  {
+    return Val{__halves2half2(toHalf(a.x), toHalf(a.y)), __halves2half2(toHalf(a.z), toHalf(a.w))};
   }
   __device__ static Val reduce3(float w0, Val v0, float w1, Val v1, float w2, Val v2)
   {

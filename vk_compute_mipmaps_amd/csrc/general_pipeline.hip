@@ -7,11 +7,11 @@
 
 namespace nvpro_pyramid {
 
-template <class F, bool THIN>
-struct GeneralShared
+template <class F>
+struct ThinShared
 {
   typename F::Tables tab;
-  typename F::Val mid[gen2MidTexels<F, THIN>()];
+  typename F::Val mid[gen2MidTexels<F, true>()];
 };
 
 template <class F>
@@ -26,67 +26,95 @@ __global__ void __launch_bounds__(kGroupBS) generalOneLevelKernel(ImageDesc img,
     generalOneGroup<F>(tab, img, inLevel, g);
 }
 
-// KX, KY: the first level's kernel sizes, or 0 (read from the image).  THIN:
-// the tile geometry (Gen2Geom) and one tile per workgroup (the grid is
-// numTiles); otherwise persistent workgroups loop over the tiles.
-template <class F, int KX, int KY, bool THIN>
-__global__ void __launch_bounds__(kGroupBS) generalTwoLevelKernel(ImageDesc img, uint32_t inLevel, uint32_t tilesX,
-                                                                uint32_t numTiles)
+// Thin tiles, one per workgroup (the grid is numTiles): straight-line code.
+// KX, KY: the first level's kernel sizes, or 0 (read from the image).
+template <class F, int KX, int KY>
+__global__ void __launch_bounds__(kGroupBS) thinTwoLevelKernel(ImageDesc img, uint32_t inLevel, uint32_t tilesX,
+                                                             uint32_t numTiles)
 {
-  __shared__ GeneralShared<F, THIN> sh;
-  if(THIN && blockIdx.x >= numTiles)  // the same for the whole workgroup
+  __shared__ ThinShared<F> sh;
+  if(blockIdx.x >= numTiles)  // the same for the whole workgroup
     return;
   const uint32_t lines = prefetchLevels(img);
   F::template fill<kGroupBS>(sh.tab, 1.0f);
   __syncthreads();
   levelsReady(lines);
-  if constexpr(THIN)  // one tile per workgroup, straight-line: ~20 fewer VGPRs than the loop
-    generalTwoGroup<F, false, KX, KY, true>(sh.tab, sh.mid, img, inLevel, tilesX, blockIdx.x);
-  else
-    for(uint32_t tile = blockIdx.x; tile < numTiles; tile += gridDim.x)
-      generalTwoGroup<F, false, KX, KY, false>(sh.tab, sh.mid, img, inLevel, tilesX, tile);
+  generalTwoGroup<F, false, KX, KY, true>(sh.tab, sh.mid, img, inLevel, tilesX, blockIdx.x);
 }
 
-// Workgroups of `kernel` that are resident on one compute unit at once.  A
-// persistent launch is capped there: more workgroups would only start after
-// the first ones had finished all their tiles.
+// One strip group per workgroup, strips of a row of groups side by side, in the
+// order of xcdContiguous: neighbouring groups share cache lines at their
+// borders, and groups in flight together read one region of memory (4095^2 and
+// 8191^2, memory accesses alone: 20.9 -> 19.2 and 73 -> 66 us).  The tables'
+// loads are issued first and the window's behind them, so that one memory round
+// trip covers both (4095x2047 15.9 -> 14.3 us, 8191^2 86 -> 78).
+using StripWide = StripGeom<8, 1>;
+
+template <class F>
+struct StripShared
+{
+  typename F::Tables tab;
+  typename F::Val border[StripWide::BORDER];
+};
+
+template <class F, int KX, int KY>
+__global__ void __launch_bounds__(StripWide::BS) __attribute__((amdgpu_waves_per_eu(4, 8)))
+stripKernel(StripStep step, uint32_t strips, uint32_t stripsInverse)
+{
+  constexpr int BS = StripWide::BS;
+  __shared__ StripShared<F> sh;
+  typename F::template TableLoads<BS> tables;
+  F::template fillLoad<BS>(tables);
+  const uint32_t unit  = xcdContiguous(blockIdx.x, gridDim.x);
+  const uint32_t block = strips == 1u ? unit : __umulhi(unit, stripsInverse);  // unit / strips
+  const StripLane L    = stripLane<StripWide>(step, unit - block * strips, block);
+  StripWindow<F, StripWide, KY> w;
+  stripLoad<F, StripWide, KY>(step, L, w);
+  F::template fillStore<BS>(sh.tab, tables, 1.0f);
+  __syncthreads();
+  stripMoved<F, StripWide, KY>(step, L, w);
+  stripCompute<F, StripWide, KX, KY>(sh.tab, sh.border, step, L, w);
+}
+
+// Workgroups of `kernel` that are resident on one compute unit at once.
 template <class K>
-static uint32_t residentPerCU(K kernel)
+static uint32_t residentPerCU(K kernel, int threads)
 {
   int n = 0;
-  if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kGroupBS, 0) != hipSuccess || n <= 0)
+  if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, 0) != hipSuccess || n <= 0)
     n = 1;
   return (uint32_t)n;
 }
 
-// A step whose thin tiles all fit on the GPU at once runs them (its time is
-// then one tile's latency, which thin tiles halve); a larger one runs the full
-// tiles, which recompute fewer border texels, on persistent workgroups.  The
-// environment variable NVPRO_PYRAMID_THIN=1 / =0 forces thin / full tiles for
-// every step (the bytes are the same either way).
+// A step whose thin tiles all fit on the GPU at once runs them: its time is then
+// one tile's latency, and a thin tile's lanes run less serial work than a
+// strip's.  A larger one runs strips.  A step with a first-level side of 1 always runs
+// thin tiles (a 65535-texel side has 529 of them).  The environment variable
+// NVPRO_PYRAMID_THIN=1 / =0 forces thin tiles / strips where both apply (the
+// bytes are the same either way).
 template <class F, int KX, int KY>
 static void launchTwoLevel(hipStream_t stream, const ImageDesc& img, uint32_t inLevel)
 {
-  static const uint32_t fit     = residentPerCU(generalTwoLevelKernel<F, KX, KY, false>);
-  static const uint32_t fitThin = residentPerCU(generalTwoLevelKernel<F, KX, KY, true>);
+  static const uint32_t fitThin = residentPerCU(thinTwoLevelKernel<F, KX, KY>, kGroupBS);
   const LevelDesc& d            = img.lv[inLevel + 2u];
-  uint32_t tilesX = 0, thinX = 0;
-  const uint32_t numTiles = generalGroupCount(d.width, d.height, 2u, F::kBytes, &tilesX);
-  const uint32_t numThin  = generalGroupCount(d.width, d.height, 2u, F::kBytes, &thinX, true);
-  const char* force       = getenv("NVPRO_PYRAMID_THIN");
-  const bool thin         = force && (force[0] == '0' || force[0] == '1')
-                                ? force[0] == '1'
-                                : (uint64_t)numThin <= (uint64_t)deviceComputeUnits() * fitThin;
-  if(thin)
-  {
-    hipLaunchKernelGGL((generalTwoLevelKernel<F, KX, KY, true>), dim3(numThin), dim3(kGroupBS), 0, stream, img,
-                       inLevel, thinX, numThin);
-    return;
-  }
-  const uint64_t cap    = (uint64_t)deviceComputeUnits() * fit;
-  const uint32_t blocks = (uint32_t)(numTiles < cap ? numTiles : cap);
-  hipLaunchKernelGGL((generalTwoLevelKernel<F, KX, KY, false>), dim3(blocks ? blocks : 1), dim3(kGroupBS), 0, stream,
-                     img, inLevel, tilesX, numTiles);
+  uint32_t thinX                = 0;
+  const uint32_t numThin = generalGroupCount(d.width, d.height, 2u, F::kBytes, &thinX, true);
+  const char* force      = getenv("NVPRO_PYRAMID_THIN");
+  const bool thin        = force && (force[0] == '0' || force[0] == '1')
+                               ? force[0] == '1'
+                               : (uint64_t)numThin <= (uint64_t)deviceComputeUnits() * fitThin;
+  if constexpr(KX != 0 && KY != 0)
+    if(!thin && stripsApply(img, inLevel))
+    {
+      const uint32_t strips  = stripCount(d.width), rows = StripWide::rows(img.lv[inLevel + 1u].height);
+      const uint32_t blocks  = (d.height + rows - 1u) / rows;
+      const uint32_t inverse = (uint32_t)((0x100000000ull + strips - 1u) / strips);
+      hipLaunchKernelGGL((stripKernel<F, KX, KY>), dim3(strips * blocks), dim3(StripWide::BS), 0, stream,
+                         stripStep(img, inLevel), strips, inverse);
+      return;
+    }
+  hipLaunchKernelGGL((thinTwoLevelKernel<F, KX, KY>), dim3(numThin), dim3(kGroupBS), 0, stream, img, inLevel, thinX,
+                     numThin);
 }
 
 template <class F>
@@ -94,7 +122,7 @@ static hipError_t launchGeneralTyped(hipStream_t stream, const ImageDesc& img, u
 {
   if(count == 1u)
   {
-    static const uint32_t oneFit = residentPerCU(generalOneLevelKernel<F>);
+    static const uint32_t oneFit = residentPerCU(generalOneLevelKernel<F>, kGroupBS);
     const LevelDesc& d           = img.lv[inLevel + 1u];
     uint32_t unused              = 0;
     const uint64_t want          = generalGroupCount(d.width, d.height, 1u, F::kBytes, &unused);

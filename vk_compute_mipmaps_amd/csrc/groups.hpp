@@ -515,7 +515,7 @@ __device__ __forceinline__ void gen2SecondLevel3(const TT& tab, const typename F
     const V h2 = waveShiftDown1(h[0]);
     if(ox < G::TX && x < l2.width && y < l2.height)
     {
-      const V v = horizontalTap<F>(axis3(l2.width), x, 3, h[0], h[1], h2);
+      const V v = horizontalTap<F>(weights3(axis3(l2.width), x), 3, h[0], h[1], h2);
       storeTexelTo<F, CO>(texelPtr(img, inLevel + 2u, x, y, F::kBytes), F::store(tab, v));
     }
   }
@@ -563,7 +563,7 @@ __device__ __forceinline__ void gen2Compute(const TT& tab, typename F::Val* mid,
         const V h2 = waveShiftDown1(h[0]);  // column 2 gx + 2, from lane + 1
         if(L.out)
         {
-          const V v = horizontalTap<F>(ax, L.gx, kx1, h[0], h[1], h2);
+          const V v = horizontalTap<F>(weights3(ax, L.gx), kx1, h[0], h[1], h2);
           storeTexel<F>(texelPtr(img, inLevel + 1u, L.gx, L.gy0 + k, F::kBytes), F::store(tab, v));
           mid[(ly0 + k) * G::MW + lane] = v;
         }
@@ -623,6 +623,326 @@ __device__ __forceinline__ void generalTwoGroupAny(const TT& tab, typename F::Va
     generalTwoGroup<F, CO, 2, 3>(tab, mid, img, inLevel, tilesX, tile);
   else
     generalTwoGroup<F, CO>(tab, mid, img, inLevel, tilesX, tile);
+}
+
+// ---------------------------------------------------------------------------
+// General pipeline, two levels, large steps: strips.
+//
+// A group is kStripCols second-level columns by a run of second-level rows,
+// G::PER to each of its G::WAVES waves, all in registers.  Lane i of every wave
+// owns second-level column x = kStripCols strip + i (lane 63 is a helper), so
+// first-level columns 2x and 2x+1 and input columns 4x..4x+3, one wide access
+// per input row; the wave's input rows are all loaded before any arithmetic.
+// The columns past a lane's own come from lane + 1 by a wave shift (the value
+// that lane computes for its first column), so every input texel is decoded
+// once per wave and every first-level texel computed once, except one
+// first-level row per group: with a 3-tall second kernel a row needs the first
+// first-level row under the next one, which the wave below hands over through
+// LDS (`border`), and the group's last wave's last row is there only for that.
+// Every value is generalSample's, from the same operands in the same order.
+// Both first-level sides must be at least 2 (so the input's at least 4).
+//
+// What bounds it (MI355X, 4095^2 sRGBA8): VALU issue (411 instructions a wave
+// of 63 x 1 second-level texels, about half of the time), the LDS lookups' bank
+// conflicts and memory each come to 50-75 % of the time.  The 31 x 7 tiles it
+// replaced (a lane per first-level column, the second level from LDS) issued
+// 50 % more VALU instructions per texel and read the input in dwords: G(0,2) of
+// 4095^2 30.1 -> 25.0 us, 8191^2 105 -> 78, 4095x2047 18.4 -> 14.2, RGBA16F
+// 22.4 -> 20.2, RGBA32F 39.1 -> 39.0; memory alone, without arithmetic, takes
+// 18, 62 and 10.3 us (4-byte texels).  Longer runs measured slower: two rows a
+// wave 26.6 / 81 / 16.7 us (88 instead of 52 VGPRs), waves marching down many
+// rows with the next rows in flight 30 / 92 / 19 (every wave then reads its own
+// far-apart rows at once).
+// ---------------------------------------------------------------------------
+constexpr uint32_t kStripCols = 63;
+
+template <uint32_t WAVES_, uint32_t PER_>
+struct StripGeom
+{
+  static constexpr uint32_t WAVES  = WAVES_, PER = PER_;
+  static constexpr uint32_t BS     = 64u * WAVES;
+  static constexpr uint32_t BORDER = (WAVES - 1u) * 2u * 64u;  // LDS values: two first-level columns per lane and boundary
+  // Second-level rows of a group, by the first level's height.
+  __host__ __device__ static uint32_t rows(uint32_t height1) { return PER * WAVES - (kernelSize(height1) == 3 ? 1u : 0u); }
+};
+
+__host__ __device__ inline uint32_t stripCount(uint32_t width2) { return (width2 + kStripCols - 1u) / kStripCols; }
+__host__ __device__ inline bool stripsApply(const ImageDesc& img, uint32_t inLevel)
+{
+  return img.lv[inLevel + 1u].width >= 2u && img.lv[inLevel + 1u].height >= 2u;
+}
+
+// The step's levels as a strip group uses them, the same for every group: for
+// the per-step kernel made on the host (one scalar load round, no level index
+// to follow).
+struct StripStep
+{
+  const uint8_t* src;
+  uint8_t *d1, *d2;  // first and second level
+  uint32_t srcPitch, pitch1, pitch2;
+  uint32_t srcWidth, srcHeight, width1, height1, width2, height2;
+  Axis3 x1, y1, x2, y2;  // axes (axis3) of the first and second level
+};
+
+__host__ __device__ inline StripStep stripStep(const ImageDesc& img, uint32_t inLevel)
+{
+  const LevelDesc &src = img.lv[inLevel], &l1 = img.lv[inLevel + 1u], &l2 = img.lv[inLevel + 2u];
+  return StripStep{img.base + src.offset, img.base + l1.offset, img.base + l2.offset, src.pitch, l1.pitch, l2.pitch,
+                   src.width, src.height, l1.width, l1.height, l2.width, l2.height, axis3(l1.width), axis3(l1.height),
+                   axis3(l2.width), axis3(l2.height)};
+}
+
+template <class F>
+struct StripRow
+{
+  typename F::Raw t[4];
+};
+
+// The input rows of one wave: four per second-level row, and one more for a
+// 3-tall kernel.
+template <class F, class G, int KY>
+struct StripWindow
+{
+  static constexpr uint32_t N = 4u * G::PER + (KY == 3 ? 1u : 0u);
+  StripRow<F> r[N];
+};
+
+struct StripLane
+{
+  uint32_t x;              // second-level column
+  uint32_t y, wave, rows;  // the wave's first second-level row, its number, and the rows it computes: the same in
+                           // the whole wave
+};
+
+template <class G>
+__device__ __forceinline__ StripLane stripLane(const StripStep& s, uint32_t strip, uint32_t block)
+{
+  constexpr uint32_t PER = G::PER;
+  const uint32_t rows = G::rows(s.height1), first = rows * block;
+  const uint32_t end  = first + rows < s.height2 ? first + rows : s.height2;
+  StripLane L;
+  L.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  L.x    = kStripCols * strip + (threadIdx.x & 63u);
+  L.y    = first + PER * L.wave;
+  L.rows = L.y < end ? (end - L.y < PER ? end - L.y : PER) : 0u;
+  return L;
+}
+
+// Loads the wave's window, a wide access per row.  The lane at the right edge,
+// x == width2, has up to three columns (it lends them, and computes first-level
+// column 2 width2 where that exists); lanes beyond it repeat its columns,
+// unused.  Its access reads up to four texels past the row's end: in the level's
+// next row (a pitch is at least a row's texels, and a row has at least four).
+// The last row has no next one: there the access is moved back into the row,
+// and stripMoved() puts the lane's columns in their places.  Rows past the last
+// repeat it, unused.  4-byte texels are read with the non-temporal hint, which
+// leaves the levels just written in the caches for the steps that read them
+// (4095x2047 chain 30.3 -> 29.1 us, 4095^2 40.6 -> 38.6); a wider texel's lanes
+// read parts of the same lines in several accesses, and with the hint read
+// memory again for each (RGBA16F G(0,2) 20.4 -> 24.2 us, RGBA32F 40 -> 68).
+template <class F, class G, int KY>
+__device__ __forceinline__ void stripLoad(const StripStep& s, const StripLane& L, StripWindow<F, G, KY>& w)
+{
+  const uint32_t at      = 4u * (L.x < s.width2 ? L.x : s.width2) * F::kBytes;
+  const uint32_t last    = (s.srcWidth - 4u) * F::kBytes;
+  const uint32_t lastRow = s.srcHeight - 1u;
+#pragma unroll
+  for(uint32_t k = 0; k < StripWindow<F, G, KY>::N; ++k)
+  {
+    const uint32_t row  = 4u * L.y + k < lastRow ? 4u * L.y + k : lastRow;  // the same in the whole wave
+    const uint32_t most = row < lastRow ? 0xffffffffu : last;
+    const uint8_t* const p = s.src + (uint64_t)row * s.srcPitch + (at < most ? at : most);
+    if constexpr(F::kBytes == 4u)
+      loadRowStream<F, 4>(p, w.r[k].t);
+    else
+      loadRow<F, 4>(p, w.r[k].t);
+  }
+}
+
+// See stripLoad: only in a group at the level's bottom right corner.
+template <class F, class G, int KY>
+__device__ __forceinline__ void stripMoved(const StripStep& s, const StripLane& L, StripWindow<F, G, KY>& w)
+{
+  constexpr uint32_t N   = StripWindow<F, G, KY>::N;
+  const uint32_t lastRow = s.srcHeight - 1u, by = 4u - (s.srcWidth & 3u);
+  const uint32_t right   = __builtin_amdgcn_readfirstlane(L.x) + 63u;
+  if(4u * L.y + N <= lastRow || right < s.width2)  // the same in the whole wave
+    return;
+  auto pick = [](bool c, typename F::Raw a, typename F::Raw b) {
+    uint32_t u[F::kBytes / 4u], v[F::kBytes / 4u];
+    __builtin_memcpy(u, &a, sizeof u);
+    __builtin_memcpy(v, &b, sizeof v);
+#pragma unroll
+    for(uint32_t i = 0; i < F::kBytes / 4u; ++i)
+      u[i] = c ? u[i] : v[i];
+    __builtin_memcpy(&a, u, sizeof u);
+    return a;
+  };
+#pragma unroll
+  for(uint32_t k = 0; k < N; ++k)
+  {
+    const bool moved = 4u * L.y + k >= lastRow && L.x >= s.width2;
+    auto& t          = w.r[k].t;
+    const typename F::Raw a = pick(by == 1u, t[1], pick(by == 2u, t[2], t[3])), b = pick(by == 1u, t[2], t[3]);
+    t[0] = pick(moved, a, t[0]);
+    t[1] = pick(moved, b, t[1]);
+    t[2] = pick(moved, t[3], t[2]);
+  }
+}
+
+// Makes v's value at this point of the program: the compiler otherwise moves
+// arithmetic whose result only a later branch uses into that branch, and keeps
+// every operand in a register until then.
+template <class V>
+__device__ __forceinline__ void settle(V& v)
+{
+  uint32_t w[sizeof(V) / 4];
+  __builtin_memcpy(w, &v, sizeof v);
+#pragma unroll
+  for(int k = 0; k < (int)(sizeof(V) / 4); ++k)
+    __asm__ volatile("" : "+v"(w[k]));
+  __builtin_memcpy(&v, w, sizeof v);
+}
+
+// First-level columns 2x and 2x+1 of the two rows under second-level row k of
+// the wave, with vertical weights wy.  Column by column, each tap of the
+// horizontal reduction added as its column is ready: the registers then hold
+// the partial sums and one column's texels.  The scheduling barriers keep the
+// compiler from starting every column's table lookups at once (twice the
+// registers).
+template <class F, class G, int KX, int KY, class TT>
+__device__ __forceinline__ void stripFirst(const TT& tab, const StripWindow<F, G, KY>& w, uint32_t k,
+                                           const Weights3 (&wy)[2], const Weights3 (&wx)[2],
+                                           typename F::Val (&out)[2][2])
+{
+  using V = typename F::Val;
+  typename F::Acc acc[2][2];
+  V lent[2], left[2];
+#pragma unroll
+  for(int j = 0; j < 4; ++j)
+  {
+    V d[5];
+#pragma unroll
+    for(uint32_t r = 0; r < (KY == 3 ? 5u : 4u); ++r)
+      d[r] = F::template load<false>(tab, w.r[4u * k + r].t[j]);
+#pragma unroll
+    for(int n = 0; n < 2; ++n)
+    {
+      const V h = verticalTap<F>(wy[n], KY, d[2 * n], d[2 * n + 1], d[KY == 3 ? 2 * n + 2 : 2 * n + 1]);
+      if constexpr(KX == 3)
+      {
+        if(j == 0)
+        {
+          lent[n]   = waveShiftDown1(h);  // column 4x + 4, from lane + 1
+          acc[n][0] = F::first3(wx[0].w0, h);
+        }
+        else if(j == 1)
+          acc[n][0] = F::next3(wx[0].w1, h, acc[n][0]);
+        else if(j == 2)
+        {
+          out[n][0] = F::done3(F::next3(wx[0].w2, h, acc[n][0]));
+          acc[n][1] = F::first3(wx[1].w0, h);
+        }
+        else
+          out[n][1] = F::done3(F::next3(wx[1].w2, lent[n], F::next3(wx[1].w1, h, acc[n][1])));
+      }
+      else
+      {
+        if(j & 1)
+          out[n][j >> 1] = reduce2<F>(left[n], h);
+        else
+          left[n] = h;
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for(int n = 0; n < 2; ++n)
+  {
+    settle(out[n][0]);
+    settle(out[n][1]);
+  }
+}
+
+// A second-level texel from first-level columns 2x and 2x+1 of rows c, a and b.
+template <class F, int KX2, int KY2>
+__device__ __forceinline__ typename F::Val stripSecond(const Weights3& wy, const Weights3& wx,
+                                                       const typename F::Val (&c)[2], const typename F::Val (&a)[2],
+                                                       const typename F::Val (&b)[2])
+{
+  using V    = typename F::Val;
+  const V g0 = verticalTap<F>(wy, KY2, c[0], a[0], b[0]), g1 = verticalTap<F>(wy, KY2, c[1], a[1], b[1]);
+  const V g2 = KX2 == 3 ? waveShiftDown1(g0) : g1;  // column 2x + 2, from lane + 1
+  return horizontalTap<F>(wx, KX2, g0, g1, g2);
+}
+
+// The group's first and second levels from the loaded rows.  CO: the second
+// level is stored with storeTexelCoherent.  Contains a barrier when the second
+// kernel is 3 tall.
+template <class F, class G, int KX, int KY, bool CO = false, class TT>
+__device__ __forceinline__ void stripCompute(const TT& tab, typename F::Val* border, const StripStep& s,
+                                             const StripLane& L, const StripWindow<F, G, KY>& w)
+{
+  using V       = typename F::Val;
+  using Raw     = typename F::Raw;
+  const int kx2 = kernelSize(s.width1), ky2 = kernelSize(s.height1);
+  const uint32_t lane = threadIdx.x & 63u;
+  constexpr uint32_t PER = G::PER;
+  const Weights3 wx1[2]  = {weights3(s.x1, 2u * L.x), weights3(s.x1, 2u * L.x + 1u)};
+  const Weights3 wx2     = weights3(s.x2, L.x);
+  const bool pair   = lane < kStripCols && L.x < s.width2;  // stores first-level columns 2x and 2x + 1
+  const bool single = L.x == s.width2 && kx2 == 3;          // stores first-level column 2x
+  uint8_t* const d1 = s.d1 + (uint64_t)(2u * L.y) * s.pitch1 + 2u * L.x * F::kBytes;
+  auto store        = [&](uint32_t k, const V(&v)[2]) {
+    const Raw q[2] = {F::store(tab, v[0]), F::store(tab, v[1])};
+    if(pair)
+      storeRow<F, 2>(d1 + (uint64_t)k * s.pitch1, q);
+    else if(single)
+      storeTexel<F>(d1 + (uint64_t)k * s.pitch1, q[0]);
+  };
+  auto second = [&](uint32_t k, const V(&c)[2], const V(&a)[2], const V(&b)[2]) {
+    const Weights3 wy = weights3(s.y2, L.y + k);
+    V v;
+    if(kx2 == 3)
+      v = ky2 == 3 ? stripSecond<F, 3, 3>(wy, wx2, c, a, b) : stripSecond<F, 3, 2>(wy, wx2, c, a, b);
+    else
+      v = ky2 == 3 ? stripSecond<F, 2, 3>(wy, wx2, c, a, b) : stripSecond<F, 2, 2>(wy, wx2, c, a, b);
+    if(pair)
+      storeTexelTo<F, CO>(s.d2 + (uint64_t)(L.y + k) * s.pitch2 + L.x * F::kBytes, F::store(tab, v));
+  };
+  // Every wave computes the first-level rows of all its PER second-level rows:
+  // past its last one the first of them is the row below it (the rest, on
+  // clamped rows, goes unused), which is stored only where it is the level's
+  // last; elsewhere the group below stores it.
+  V first[PER][2][2];
+#pragma unroll
+  for(uint32_t k = 0; k < PER; ++k)
+  {
+    const uint32_t y      = 2u * (L.y + k);
+    const Weights3 wy1[2] = {weights3(s.y1, y), weights3(s.y1, y + 1u)};
+    stripFirst<F, G, KX, KY>(tab, w, k, wy1, wx1, first[k]);
+    if(k == 0u && ky2 == 3 && L.wave != 0u)
+#pragma unroll
+      for(int j = 0; j < 2; ++j)
+        border[((L.wave - 1u) * 2u + j) * 64u + lane] = first[0][0][j];
+    if(k < L.rows || (ky2 == 3 && y == 2u * s.height2))
+      store(2u * k, first[k][0]);
+    if(k < L.rows)
+      store(2u * k + 1u, first[k][1]);
+    if(k > 0u && k <= L.rows)
+      second(k - 1u, first[k - 1u][0], first[k - 1u][1], first[k][0]);
+  }
+  if(ky2 == 3)
+    __syncthreads();
+  if(L.rows == PER)
+  {
+    V under[2] = {first[0][0][0], first[0][0][1]};
+    if(ky2 == 3)
+#pragma unroll
+      for(int j = 0; j < 2; ++j)
+        under[j] = border[(L.wave * 2u + j) * 64u + lane];
+    second(PER - 1u, first[PER - 1u][0], first[PER - 1u][1], under);
+  }
 }
 
 // ---------------------------------------------------------------------------
