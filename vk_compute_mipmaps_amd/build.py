@@ -45,6 +45,8 @@ HIPCC_FLAGS = [
     "-fPIC",
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # Leading scalar arguments of a kernel arrive in scalar registers.
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",
     "-Wall",
     "-Wno-unused-function",
 ]

@@ -18,6 +18,8 @@
 //                        from (box, reduce2, reduce3 below)
 //   Acc, first3, next3,  reduce3 tap by tap: done3(next3(w2, v2, next3(w1, v1,
 //   done3                first3(w0, v0)))) is reduce3(w0, v0, w1, v1, w2, v2)
+//   Chan, chanRaw,       one channel of a Val (a Val is four in memory order), of a
+//   chanStore, chanLoad  Raw, and NVPRO_PYRAMID_STORE / _LOAD of channel c alone
 //   kPrescale            whether load<true> then box<true> equals box<false>
 //                        of plain loads bit for bit (exact scaling by 0.25)
 //
@@ -79,7 +81,8 @@ struct Fp32Arith
   {
     return fma3(w0, v0, w1, v1, w2, v2);
   }
-  using Acc = float4;
+  using Chan = float;
+  using Acc  = float4;
   __device__ static Acc first3(float w, Val v) { return f4mul(v, w); }
   __device__ static Acc next3(float w, Val v, Acc a)
   {
@@ -167,10 +170,11 @@ struct Srgba8 : Fp32Arith
   template <int BS>
   __device__ static uint32_t encWord(int k)
   {
-    constexpr uint32_t N = NVPRO_SRGB_ENC_BUCKETS / 4u, spare = TableLoads<BS>::kEnc * BS - N;
-    static_assert(spare <= N, "every thread has a word");
-    const uint32_t i = threadIdx.x + k * BS;
-    return i < N ? i : i - spare;
+    constexpr uint32_t N = NVPRO_SRGB_ENC_BUCKETS / 4u;
+    static_assert(BS <= 3 * N, "at most two words past the table's end");
+    uint32_t i = threadIdx.x + k * BS;
+    i          = i < N ? i : i - N;
+    return i < N ? i : i - N;
   }
   template <int BS>
   __device__ static void fillLoad(TableLoads<BS>& r)
@@ -279,6 +283,15 @@ struct Srgba8 : Fp32Arith
   }
   __device__ static uint32_t encodeChannel(const Tables& t, float x) { return encodeHigh(t, x) >> 16; }
 
+  using ChanRaw = uint8_t;
+  __device__ static ChanRaw chanStore(const Tables& t, float v, uint32_t c)
+  {
+    const uint32_t rgb = encodeChannel(t, v);
+    const uint32_t a   = (uint32_t)__builtin_amdgcn_fmed3f(v + 0.5f, 0.0f, 255.0f);
+    return (ChanRaw)(c == 3u ? a : rgb);
+  }
+  __device__ static float chanLoad(const Tables& t, ChanRaw q, uint32_t c) { return c == 3u ? (float)q : t.dec[q]; }
+
   // srgbFromLinearVec (preamble:123-128); alpha (code units) = floor(a + 0.5)
   // clamped to [0, 255].  Byte selectors of v_perm_b32: 0-3 the second
   // operand's bytes, 4-7 the first's, 12 zero.
@@ -335,6 +348,9 @@ struct Rgba32f : Fp32Arith
   {
     return Raw{v.x, v.y, v.z, v.w};
   }
+  using ChanRaw = float;
+  __device__ static ChanRaw chanStore(const Tables&, float v, uint32_t) { return v; }
+  __device__ static float chanLoad(const Tables&, ChanRaw q, uint32_t) { return q; }
 };
 
 // ---------------------------------------------------------------------------
@@ -384,6 +400,9 @@ struct Rgba16f : Fp32Arith
   {
     return Raw{f2h(v.x) | f2h(v.y) << 16, f2h(v.z) | f2h(v.w) << 16};
   }
+  using ChanRaw = uint16_t;
+  __device__ static ChanRaw chanStore(const Tables&, float v, uint32_t) { return (ChanRaw)f2h(v); }
+  __device__ static float chanLoad(const Tables&, ChanRaw q, uint32_t) { return h2f(q); }
 };
 
 // ---------------------------------------------------------------------------
@@ -439,6 +458,10 @@ struct Rgba16fPacked
     const __half2 k = __float2half2_rn(s);  // 0.25 and 0.5 are exact in binary16
     return Val{__hmul2(a.rg, k), __hmul2(a.ba, k)};
   }
+  using Chan    = _Float16;
+  using ChanRaw = _Float16;
+  __device__ static ChanRaw chanStore(const Tables&, Chan v, uint32_t) { return v; }
+  __device__ static Chan chanLoad(const Tables&, ChanRaw q, uint32_t) { return q; }
   using Acc = float4;
   __device__ static float4 widen(Val v)
   {
@@ -457,6 +480,33 @@ struct Rgba16fPacked
     const float2 b0 = __half22float2(v0.ba), b1 = __half22float2(v1.ba), b2 = __half22float2(v2.ba);
     return Val{__halves2half2(toHalf(fma3(w0, a0.x, w1, a1.x, w2, a2.x)), toHalf(fma3(w0, a0.y, w1, a1.y, w2, a2.y))),
                __halves2half2(toHalf(fma3(w0, b0.x, w1, b1.x, w2, b2.x)), toHalf(fma3(w0, b0.y, w1, b1.y, w2, b2.y)))};
+  }
+};
+
+// One channel of F as a value of its own: the same operations, in the same
+// arithmetic, as F's on that channel.
+template <class Chan>
+struct ChannelArith;
+template <>
+struct ChannelArith<float>
+{
+  using Val = float;
+  __device__ static Val add(Val a, Val b) { return a + b; }
+  __device__ static Val mul(Val a, float s) { return a * s; }
+  __device__ static Val reduce3(float w0, Val v0, float w1, Val v1, float w2, Val v2)
+  {
+    return fma3(w0, v0, w1, v1, w2, v2);
+  }
+};
+template <>
+struct ChannelArith<_Float16>
+{
+  using Val = _Float16;
+  __device__ static Val add(Val a, Val b) { return a + b; }
+  __device__ static Val mul(Val a, float s) { return a * (_Float16)s; }
+  __device__ static Val reduce3(float w0, Val v0, float w1, Val v1, float w2, Val v2)
+  {
+    return __builtin_bit_cast(_Float16, toHalf(fma3(w0, (float)v0, w1, (float)v1, w2, (float)v2)));
   }
 };
 

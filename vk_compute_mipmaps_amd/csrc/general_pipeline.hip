@@ -194,6 +194,17 @@ static uint64_t firstOutput(const ImageDesc& img, const NvproPyramidStep& s)
   return (uint64_t)first.width * first.height;
 }
 
+// Whether each of the steps from `first` on starts at the level the one before
+// it ends with, as the dispatcher loop's own steps do (a custom dispatcher may
+// record others): a tail hands its levels on without reading them back.
+static bool consecutive(const NvproPyramidStep* steps, uint32_t first, uint32_t count)
+{
+  for(uint32_t k = first; k + 1u < count; ++k)
+    if(steps[k + 1u].inputLevel != steps[k].inputLevel + steps[k].levelCount)
+      return false;
+  return true;
+}
+
 // Persistent workgroups per compute unit of a fast step of `groups` groups
 // (measured on MI355X, sRGBA8 F(0,6), per-step time): up to 16 groups per
 // compute unit, 8 (the most that fit: 4096^2 22.3 us; with 4 or 3, 22.6-22.8);
@@ -240,7 +251,7 @@ hipError_t executePlan(hipStream_t stream, const ImageDesc& img, const NvproPyra
     const NvproPyramidStep& s = steps[i];
     // The one-workgroup tail pays off when it saves launches: with a single step
     // left, that step's own kernel is as quick.
-    if(firstOutput(img, s) <= kTailMaxTexels && count - i >= 2u)
+    if(firstOutput(img, s) <= kTailMaxTexels && count - i >= 2u && consecutive(steps, i, count))
     {
       ++*launches;
       return launchTail(stream, img, tailFrom(steps, i, count));
