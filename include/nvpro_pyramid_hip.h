@@ -143,8 +143,12 @@ uint32_t nvproPyramidDefaultGeneralDispatcher(NvproPyramidCmd* cmd, const NvproP
  * texels run in one launch, and a fast step (of at most 64 or at least 1024
  * workgroups) whose successor is a fast step of one workgroup, or the rest of
  * the plan with at most 128 texels in its first output level, runs that in its
- * own launch, in whichever workgroup finishes last.  Results are the same bytes
- * either way.  This fusion needs a 16.6 KB block of arrival counters per
+ * own launch, in whichever workgroup finishes last.  Two steps or more of at
+ * most four levels together, small enough that tiles of at most 4x4 texels of
+ * their last level are no more than the compute units, run in one launch too;
+ * sRGBA8 steps that a general step begins do so only where the second could be
+ * in the last launch.  Results are the same bytes either way.  Running a
+ * successor in a step's own launch needs a 16.6 KB block of arrival counters per
  * stream, taken from a static device array of 64 blocks per device (nothing is
  * allocated; a stream that fuses keeps its block until nvproPyramidStreamRelease
  * or the end of the process, and while 64 streams of a device hold one, others

@@ -284,6 +284,14 @@ hipError_t executePlan(hipStream_t stream, const ImageDesc& img, const NvproPyra
         return launchFast(stream, img, s.inputLevel, s.levelCount, fastWorkgroupsPerCU(img, s), &next, &tail);
       }
     }
+    uint32_t tileX = 0, tileY = 0;
+    if(const uint32_t n = tileSteps(img, steps + i, count - i, &tileX, &tileY))
+    {
+      if(hipError_t e = launchTiles(stream, img, tailFrom(steps, i, i + n), tileX, tileY))
+        return e;
+      i += n - 1u;
+      continue;
+    }
     hipError_t e = fast ? launchFast(stream, img, s.inputLevel, s.levelCount, fastWorkgroupsPerCU(img, s))
                         : launchGeneral(stream, img, s.inputLevel, s.levelCount);
     if(e != hipSuccess)

@@ -128,6 +128,13 @@ hipError_t launchFast(hipStream_t stream, const ImageDesc& img, uint32_t inputLe
                       uint32_t wavesPerCU, const NextStep* next = nullptr, const TailPlan* tail = nullptr);
 hipError_t launchGeneral(hipStream_t stream, const ImageDesc& img, uint32_t inputLevel, uint32_t levelCount);
 hipError_t launchTail(hipStream_t stream, const ImageDesc& img, const TailPlan& plan);
+// The same steps in one launch of tiles (at most kTileSide x kTileSide texels of
+// the last of at most kTileLevels levels), one workgroup each, where that pays:
+// how many of `steps` it takes (0: none) and the tile.
+constexpr uint32_t kTileLevels = 4, kTileSide = 4;
+uint32_t tileSteps(const ImageDesc& img, const NvproPyramidStep* steps, uint32_t count, uint32_t* tileX,
+                   uint32_t* tileY);
+hipError_t launchTiles(hipStream_t stream, const ImageDesc& img, const TailPlan& plan, uint32_t tileX, uint32_t tileY);
 
 // Batched kernel over items [itemBegin, itemEnd) of a work list in device
 // memory.  queue: one persistent launch that dequeues items and waits on their
@@ -174,8 +181,9 @@ hipError_t launchSynthBatch(hipStream_t stream, const SynthJob* jobs, const Synt
 uint32_t appendSynthChunks(std::vector<SynthChunk>& chunks, uint32_t job, uint32_t width, uint32_t height,
                            uint64_t texelsPerChunk);
 
-// Launch a validated plan: per-step kernels for the large steps, then one tail
-// launch for the small remainder.  With `arrive` (kArriveWords zeroed counters
+// Launch a validated plan: per-step kernels for the large steps, one launch of
+// tiles for a run of short ones after them, then one tail launch for the small
+// remainder.  With `arrive` (kArriveWords zeroed counters
 // of the stream), a fast step whose successor is a fast step of one group, or
 // a tail of at most kFastTailTexels first outputs, runs that successor in its
 // own launch.  *launches: the kernel launches made.
