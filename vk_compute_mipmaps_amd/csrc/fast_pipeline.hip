@@ -59,44 +59,92 @@ struct FastShared
 // bodies load with.
 static_assert(2u * kFastTailTexels <= (uint32_t)kGroupBS, "tail ping-pong fits the level-2 scratch");
 
-// NT: the step's input loads carry the non-temporal hint.
+// The groups of a step that this workgroup has, as both kernels below run them.
+// The first group's loads are issued behind the tables', so that one memory
+// round trip covers both.  NT: the input loads carry the non-temporal hint.
+// Returns how many groups it ran.
 template <class F, int COUNT, bool CONT, bool NT>
-__global__ void __launch_bounds__(kGroupBS) __attribute__((amdgpu_waves_per_eu(F::kBytes > 8u ? 4 : 8, 8)))
-fastPipelineKernel(ImageDesc img, uint32_t inLevel, uint32_t tilesX, uint32_t numTiles, NextStep next, TailPlan tail)
+__device__ __forceinline__ uint32_t fastGroups(FastShared<F, COUNT, CONT>& sh, const uint8_t* src, uint32_t pitch,
+                                               const FastTilesInverse& tiles, uint32_t blocks,
+                                               const FastOut<COUNT, true>& out, uint32_t lines)
 {
-  __shared__ FastShared<F, COUNT, CONT> sh;
-  const uint32_t lines = prefetchLevels(img);
-  F::template fill<kGroupBS>(sh.tab, F::kPrescale ? 0.25f : 1.0f);
+  constexpr bool STRIP     = COUNT == 6;
+  constexpr bool TABLES    = F::kBytes == 4u;  // the other formats have none to overlap, and no registers to spare
+  const uint32_t numGroups = (tiles.count + FastGeom<COUNT>::TILES_PER_WG - 1u) / FastGeom<COUNT>::TILES_PER_WG;
+  typename F::template TableLoads<kGroupBS> tables;
+  F::template fillLoad<kGroupBS>(tables);
+  FastWindow<F, COUNT> w;
+  uint32_t g = blockIdx.x, iter = 0;
+  // The successor's index arithmetic is not to be shared with this: it would be
+  // held in registers, or spilled, over the whole loop.
+  uint32_t thread = threadIdx.x;
+  __asm__ volatile("" : "+v"(thread));
+  if constexpr(TABLES)
+    fastLoad<F, COUNT, STRIP, NT>(src, pitch, tiles, g, thread, w);
+  out.ready();
+  F::template fillStore<kGroupBS>(sh.tab, tables, F::kPrescale ? 0.25f : 1.0f);
   __syncthreads();
   levelsReady(lines);
-  const uint32_t numGroups = (numTiles + FastGeom<COUNT>::TILES_PER_WG - 1u) / FastGeom<COUNT>::TILES_PER_WG;
-  uint32_t iter            = 0;
-  for(uint32_t g = blockIdx.x; g < numGroups; g += gridDim.x, ++iter)
-    fastGroup<F, COUNT, CONT, COUNT == 6, NT>(sh.tab, sh.level2, img, inLevel, tilesX, numTiles, g, iter);
-  if constexpr(CONT)
+  for(;;)
   {
-    if(!arriveLast(next.arrive, gridDim.x, reinterpret_cast<uint32_t*>(sh.level2)))
-      return;
-    if(next.kind == kNextTail)
+    if constexpr(!TABLES)
+      fastLoad<F, COUNT, STRIP, NT>(src, pitch, tiles, g, thread, w);
+    fastCompute<F, COUNT, CONT, STRIP>(sh.tab, sh.level2, out, tiles, g, iter, thread, w);
+    g += blocks;
+    ++iter;
+    if(g >= numGroups)
+      return iter;
+    if constexpr(TABLES)
+      fastLoad<F, COUNT, STRIP, NT>(src, pitch, tiles, g, thread, w);
+  }
+}
+
+// The leading scalar arguments are in registers at the start (build.py's
+// kernarg-preload-count), so that the first loads wait for no argument, and all
+// of them are 96 bytes: a launch with more than that costs the host another
+// 0.7 us.  With both, chains of 256^2, 1024^2 and 2560x1440 sRGBA8 went from
+// 6.4, 8.2 and 16.2 us to 6.2, 7.2 and 13.3.
+template <class F, int COUNT, bool NT>
+__global__ void __launch_bounds__(kGroupBS) __attribute__((amdgpu_waves_per_eu(F::kBytes > 8u ? 4 : 8, 8)))
+fastPipelineKernel(const uint8_t* src, uint32_t pitch, uint32_t numTiles, uint32_t tilesInverse, uint16_t tilesX,
+                   uint16_t blocks, FastOut<COUNT, true> out)
+{
+  __shared__ FastShared<F, COUNT, false> sh;
+  fastGroups<F, COUNT, false, NT>(sh, src, pitch, FastTilesInverse{tilesX, numTiles, tilesInverse}, blocks, out, 0u);
+}
+
+// The same and then, in the last workgroup, the successor (a NextStep's fields).
+template <class F, int COUNT, bool NT>
+__global__ void __launch_bounds__(kGroupBS) __attribute__((amdgpu_waves_per_eu(F::kBytes > 8u ? 4 : 8, 8)))
+fastFusedKernel(const uint8_t* src, uint32_t pitch, uint32_t numTiles, uint32_t tilesInverse, uint16_t tilesX,
+                uint16_t blocks, uint32_t* arrive, uint32_t nextKind, uint32_t nextLevel, uint32_t nextCount,
+                uint32_t nextTilesX, uint32_t nextTiles, FastOut<COUNT, true> out, ImageDesc img, TailPlan tail)
+{
+  __shared__ FastShared<F, COUNT, true> sh;
+  const uint32_t lines = prefetchLevels(img);
+  const FastTilesInverse tiles{tilesX, numTiles, tilesInverse};
+  const uint32_t iter = fastGroups<F, COUNT, true, NT>(sh, src, pitch, tiles, blocks, out, lines);
+  if(!arriveLast(arrive, blocks, reinterpret_cast<uint32_t*>(sh.level2)))
+    return;
+  if(nextKind == kNextTail)
+  {
+    if(F::kPrescale)
     {
-      if(F::kPrescale)
-      {
-        F::template fill<kGroupBS>(sh.tab, 1.0f);
-        __syncthreads();
-      }
-      tailRun<F, kGroupBS, 1, false>(sh.tab, sh.level2, sh.level2 + kFastTailTexels, img, tail);
-      return;
+      F::template fill<kGroupBS>(sh.tab, 1.0f);
+      __syncthreads();
     }
-    switch(next.count)
-    {
-      case 1: fastGroup<F, 1>(sh.tab, sh.level2, img, next.inLevel, next.tilesX, next.numTiles, 0u, iter); break;
-      case 2: fastGroup<F, 2>(sh.tab, sh.level2, img, next.inLevel, next.tilesX, next.numTiles, 0u, iter); break;
-      case 3: fastGroup<F, 3>(sh.tab, sh.level2, img, next.inLevel, next.tilesX, next.numTiles, 0u, iter); break;
-      case 4: fastGroup<F, 4>(sh.tab, sh.level2, img, next.inLevel, next.tilesX, next.numTiles, 0u, iter); break;
-      case 5: fastGroup<F, 5>(sh.tab, sh.level2, img, next.inLevel, next.tilesX, next.numTiles, 0u, iter); break;
-      case 6: fastGroup<F, 6>(sh.tab, sh.level2, img, next.inLevel, next.tilesX, next.numTiles, 0u, iter); break;
-      default: break;
-    }
+    tailRun<F, kGroupBS, 1, false>(sh.tab, sh.level2, sh.level2 + kFastTailTexels, img, tail);
+    return;
+  }
+  switch(nextCount)
+  {
+    case 1: fastGroup<F, 1>(sh.tab, sh.level2, img, nextLevel, nextTilesX, nextTiles, 0u, iter); break;
+    case 2: fastGroup<F, 2>(sh.tab, sh.level2, img, nextLevel, nextTilesX, nextTiles, 0u, iter); break;
+    case 3: fastGroup<F, 3>(sh.tab, sh.level2, img, nextLevel, nextTilesX, nextTiles, 0u, iter); break;
+    case 4: fastGroup<F, 4>(sh.tab, sh.level2, img, nextLevel, nextTilesX, nextTiles, 0u, iter); break;
+    case 5: fastGroup<F, 5>(sh.tab, sh.level2, img, nextLevel, nextTilesX, nextTiles, 0u, iter); break;
+    case 6: fastGroup<F, 6>(sh.tab, sh.level2, img, nextLevel, nextTilesX, nextTiles, 0u, iter); break;
+    default: break;
   }
 }
 
@@ -113,25 +161,29 @@ static void launchFastCount(hipStream_t stream, const ImageDesc& img, uint32_t i
   const LevelDesc& in     = img.lv[inLevel];
   const uint32_t tilesX   = in.width >> COUNT, tilesY = in.height >> COUNT;
   const uint64_t groups   = fastGroupCount(in.width, in.height, COUNT);
-  const uint64_t cap      = (uint64_t)deviceComputeUnits() * wgPerCU;
+  const uint64_t cap      = min((uint64_t)deviceComputeUnits() * wgPerCU, (uint64_t)0xffffu);
   const uint32_t blocks   = (uint32_t)(groups < cap ? groups : cap);
-  const TailPlan none{};
-  const dim3 grid(blocks ? blocks : 1), wg(kGroupBS);
+  const dim3 grid(blocks), wg(kGroupBS);
+  const uint32_t inverse = (uint32_t)((0x100000000ull + tilesX - 1u) / tilesX);
+  FastOut<COUNT, true> out;
+  for(int r = 0; r < COUNT; ++r)
+  {
+    out.base[r]  = img.base + img.lv[inLevel + 1u + (uint32_t)r].offset;
+    out.pitch[r] = img.lv[inLevel + 1u + (uint32_t)r].pitch;
+  }
   // Non-temporal input loads for 6-level steps in the kNtMin..kNtMaxGroupsPerCU range.
+  constexpr bool NT  = COUNT == 6;
   const uint64_t cus = deviceComputeUnits();
-  const bool nt      = COUNT == 6 && groups >= kNtMinGroupsPerCU * cus && groups <= kNtMaxGroupsPerCU * cus;
-  if(next && nt)
-    hipLaunchKernelGGL((fastPipelineKernel<F, COUNT, true, COUNT == 6>), grid, wg, 0, stream, img, inLevel, tilesX,
-                       tilesX * tilesY, *next, tail ? *tail : none);
-  else if(next)
-    hipLaunchKernelGGL((fastPipelineKernel<F, COUNT, true, false>), grid, wg, 0, stream, img, inLevel, tilesX,
-                       tilesX * tilesY, *next, tail ? *tail : none);
-  else if(nt)
-    hipLaunchKernelGGL((fastPipelineKernel<F, COUNT, false, COUNT == 6>), grid, wg, 0, stream, img, inLevel, tilesX,
-                       tilesX * tilesY, NextStep{}, none);
+  const bool nt      = NT && groups >= kNtMinGroupsPerCU * cus && groups <= kNtMaxGroupsPerCU * cus;
+  auto launch       = [&](auto kernel, auto... more) {
+    hipLaunchKernelGGL(kernel, grid, wg, 0, stream, img.base + in.offset, in.pitch, tilesX * tilesY, inverse,
+                       (uint16_t)tilesX, (uint16_t)blocks, more...);
+  };
+  if(next)
+    launch(nt ? fastFusedKernel<F, COUNT, NT> : fastFusedKernel<F, COUNT, false>, next->arrive, next->kind,
+           next->inLevel, next->count, next->tilesX, next->numTiles, out, img, tail ? *tail : TailPlan{});
   else
-    hipLaunchKernelGGL((fastPipelineKernel<F, COUNT, false, false>), grid, wg, 0, stream, img, inLevel, tilesX,
-                       tilesX * tilesY, NextStep{}, none);
+    launch(nt ? fastPipelineKernel<F, COUNT, NT> : fastPipelineKernel<F, COUNT, false>, out);
 }
 
 template <class F>

@@ -87,6 +87,20 @@ __host__ __device__ inline uint32_t fastGroupCount(uint32_t width, uint32_t heig
   return (tiles + perWG - 1u) / perWG;
 }
 
+// The tiles of a fast step: `x` in a row, `count` in all; row(tile) is
+// tile / x, by multiplication where the host prepared the inverse (2^32 / x,
+// rounded up: exact while tile * x < 2^32).
+struct FastTiles
+{
+  uint32_t x, count;
+  __device__ __forceinline__ uint32_t row(uint32_t tile) const { return tile / x; }
+};
+struct FastTilesInverse
+{
+  uint32_t x, count, inverse;
+  __device__ __forceinline__ uint32_t row(uint32_t tile) const { return x == 1u ? tile : __umulhi(tile, inverse); }
+};
+
 // The input block of one lane for group g of a fast step: its 2^LB rows, all
 // loads issued before any arithmetic.
 template <class F, int COUNT>
@@ -95,34 +109,33 @@ struct FastWindow
   typename F::Raw raw[1 << FastGeom<COUNT>::LB][1 << FastGeom<COUNT>::LB];
 };
 
-// NT: load with the non-temporal hint (data read once).
-template <class F, int COUNT, bool STRIP, bool NT = false>
-__device__ __forceinline__ void fastLoad(const ImageDesc& img, uint32_t inLevel, uint32_t tilesX, uint32_t numTiles,
-                                         uint32_t g, FastWindow<F, COUNT>& w)
+// NT: load with the non-temporal hint (data read once).  thread: threadIdx.x.
+template <class F, int COUNT, bool STRIP, bool NT, class Tiles>
+__device__ __forceinline__ void fastLoad(const uint8_t* src, uint32_t pitch, const Tiles& tiles, uint32_t g,
+                                         uint32_t thread, FastWindow<F, COUNT>& w)
 {
   using G           = FastGeom<COUNT>;
   constexpr int LB  = G::LB;
   constexpr int BLK = 1 << LB;
   uint32_t tig, px, py;
-  fastLanePos<COUNT, STRIP>(threadIdx.x, tig, px, py);
-  const uint32_t tile = g * G::TILES_PER_WG + tig;
-  if(tile >= numTiles)
-    return;
-  const uint32_t ty = tile / tilesX, tx = tile - ty * tilesX;
+  fastLanePos<COUNT, STRIP>(thread, tig, px, py);
+  uint32_t tile = g * G::TILES_PER_WG + tig;
+  if(G::TILES_PER_WG > 1)  // no branch around the loads: lanes past the last tile read its texels, unused
+    tile = tile < tiles.count ? tile : tiles.count - 1u;
+  const uint32_t ty = tiles.row(tile), tx = tile - ty * tiles.x;
   const uint32_t x0 = (tx << COUNT) + (px << LB), y0 = (ty << COUNT) + (py << LB);
-  const LevelDesc& in = img.lv[inLevel];
-  const uint8_t* p    = img.base + in.offset + (uint64_t)y0 * in.pitch + (uint64_t)x0 * F::kBytes;
+  const uint8_t* p  = src + (uint64_t)y0 * pitch + (uint64_t)x0 * F::kBytes;
   if constexpr(NT)
   {
 #pragma unroll
     for(int r = 0; r < BLK; ++r)
-      loadRowStream<F, BLK>(p + (uint64_t)r * in.pitch, w.raw[r]);
+      loadRowStream<F, BLK>(p + (uint64_t)r * pitch, w.raw[r]);
   }
   else
   {
 #pragma unroll
     for(int r = 0; r < BLK; ++r)
-      loadRow<F, BLK>(p + (uint64_t)r * in.pitch, w.raw[r]);
+      loadRow<F, BLK>(p + (uint64_t)r * pitch, w.raw[r]);
   }
 }
 
@@ -141,6 +154,7 @@ struct FastOut
   uint8_t* base[COUNT];
   uint32_t pitch[COUNT];
 
+  FastOut() = default;
   __device__ __forceinline__ FastOut(const ImageDesc& img, uint32_t inLevel)
   {
 #pragma unroll
@@ -149,8 +163,14 @@ struct FastOut
       const LevelDesc& d = img.lv[inLevel + 1u + (uint32_t)r];
       base[r]            = img.base + d.offset;
       pitch[r]           = d.pitch;
-      __asm__ volatile("" ::"s"(base[r]), "s"(pitch[r]));
     }
+    ready();
+  }
+  __device__ __forceinline__ void ready() const
+  {
+#pragma unroll
+    for(int r = 0; r < COUNT; ++r)
+      __asm__ volatile("" ::"s"(base[r]), "s"(pitch[r]));
   }
   // Texel (x, y) of level inLevel + r, r in 1..COUNT.
   __device__ __forceinline__ uint8_t* at(int r, uint32_t x, uint32_t y, uint32_t bytes) const
@@ -172,14 +192,12 @@ struct FastOut<COUNT, false>
   }
 };
 
-// Group g of a fast step of `img` from level inLevel (tilesX x tilesY tiles in
-// all, numTiles = their product), from the lane blocks fastLoad put in `w`.
-// `level2`: kGroupBS values of LDS scratch (unused when COUNT < 3).  Contains
-// barriers when COUNT >= 3.
-template <class F, int COUNT, bool CO, bool STRIP, bool HOIST, class TT>
-__device__ __forceinline__ void fastCompute(const TT& tab, typename F::Val* level2, const ImageDesc& img,
-                                            uint32_t inLevel, uint32_t tilesX, uint32_t numTiles, uint32_t g,
-                                            uint32_t iter, const FastWindow<F, COUNT>& w)
+// Group g of a fast step with output levels `out`, from the lane blocks
+// fastLoad put in `w`.  `level2`: kGroupBS values of LDS scratch (unused when
+// COUNT < 3).  Contains barriers when COUNT >= 3.
+template <class F, int COUNT, bool CO, bool STRIP, class TT, class Out, class Tiles>
+__device__ __forceinline__ void fastCompute(const TT& tab, typename F::Val* level2, const Out& out, const Tiles& tiles,
+                                            uint32_t g, uint32_t iter, uint32_t thread, const FastWindow<F, COUNT>& w)
 {
   using G            = FastGeom<COUNT>;
   using Raw          = typename F::Raw;
@@ -188,18 +206,17 @@ __device__ __forceinline__ void fastCompute(const TT& tab, typename F::Val* leve
   constexpr int BLK  = 1 << LB;
   constexpr bool PRE = F::kPrescale;
 
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t wave = threadIdx.x >> 6;
+  const uint32_t lane = thread & 63u;
+  const uint32_t wave = thread >> 6;
   uint32_t tig, px, py;
-  fastLanePos<COUNT, STRIP>(threadIdx.x, tig, px, py);
-  const FastOut<COUNT, HOIST> out(img, inLevel);
+  fastLanePos<COUNT, STRIP>(thread, tig, px, py);
 
   // Levels 1 and 2 of this thread's block.
   const uint32_t tile = g * G::TILES_PER_WG + tig;
   V v{};
-  if(tile < numTiles)  // whole tiles
+  if(tile < tiles.count)  // whole tiles
   {
-    const uint32_t ty = tile / tilesX, tx = tile - ty * tilesX;
+    const uint32_t ty = tiles.row(tile), tx = tile - ty * tiles.x;
     const uint32_t x0 = (tx << COUNT) + (px << LB), y0 = (ty << COUNT) + (py << LB);
     const auto& raw = w.raw;
 
@@ -233,7 +250,7 @@ __device__ __forceinline__ void fastCompute(const TT& tab, typename F::Val* leve
   if constexpr(G::UPPER)
   {
     __syncthreads();  // the previous duty wave has read level2[]
-    level2[threadIdx.x] = v;
+    level2[thread] = v;
     __syncthreads();
     if(wave == (iter & 3u))
     {
@@ -247,9 +264,9 @@ __device__ __forceinline__ void fastCompute(const TT& tab, typename F::Val* leve
       const uint32_t b  = STRIP ? 2u * qy * (uint32_t)G::RW + (lane >> TEAM3) * (uint32_t)G::T + 2u * qx : 4u * lane;
       const uint32_t dy = STRIP ? (uint32_t)G::RW : 2u;
       V u = box<F, false>(level2[b], level2[b + 1u], level2[b + dy], level2[b + dy + 1u], fastOrder(COUNT, 3u));
-      if(t3 < numTiles)
+      if(t3 < tiles.count)
       {
-        const uint32_t ty = t3 / tilesX, tx = t3 - ty * tilesX;
+        const uint32_t ty = tiles.row(t3), tx = t3 - ty * tiles.x;
         storeTexelTo<F, CO && COUNT == 3>(out.at(3, (tx << (COUNT - 3)) + qx, (ty << (COUNT - 3)) + qy, F::kBytes),
                                           F::store(tab, u));
 #pragma unroll
@@ -291,9 +308,12 @@ __device__ __forceinline__ void fastGroup(const TT& tab, typename F::Val* level2
                                           uint32_t inLevel, uint32_t tilesX, uint32_t numTiles, uint32_t g,
                                           uint32_t iter)
 {
+  const LevelDesc& in = img.lv[inLevel];
+  const FastTiles tiles{tilesX, numTiles};
+  const FastOut<COUNT, HOIST> out(img, inLevel);
   FastWindow<F, COUNT> w;
-  fastLoad<F, COUNT, STRIP, NT>(img, inLevel, tilesX, numTiles, g, w);
-  fastCompute<F, COUNT, CO, STRIP, HOIST>(tab, level2, img, inLevel, tilesX, numTiles, g, iter, w);
+  fastLoad<F, COUNT, STRIP, NT>(img.base + in.offset, in.pitch, tiles, g, threadIdx.x, w);
+  fastCompute<F, COUNT, CO, STRIP>(tab, level2, out, tiles, g, iter, threadIdx.x, w);
 }
 
 // ---------------------------------------------------------------------------
