@@ -148,11 +148,19 @@ fastFusedKernel(const uint8_t* src, uint32_t pitch, uint32_t numTiles, uint32_t 
   }
 }
 
-// Groups per compute unit for which 6-level steps load their input with the
-// non-temporal hint (measured on MI355X, sRGBA8 F(0,6), 4096^2 at 16 groups per
-// unit: 22.4 -> 20.3 us; 16384^2 at 256 per unit, on 3 workgroups per unit:
-// 291 -> 302 us).
-constexpr uint64_t kNtMinGroupsPerCU = 8, kNtMaxGroupsPerCU = 16;
+// Whether a fast step of `groups` groups loads its input with the non-temporal
+// hint: sRGBA8 steps of more than one group and up to 64 per compute unit (an
+// input of up to 256 MiB), whose input then leaves the caches to the levels
+// being written.  Measured on MI355X, us per chain over images that are not in
+// any cache, without and with: 1920x1080 13.3 and 12.9, 2048^2 11.5 and 11.1,
+// 4096^2 25.0 and 22.7, 8192x4096 47.0 and 41.4, 8192^2 (64 groups) 88 and 74;
+// beyond, 10240^2 122 and 127, 16384^2 304 and 324.  Wider texels are slower
+// with it at every size (RGBA16F 8192^2 140 and 152, RGBA32F 4096^2 69 and 95).
+bool fastInputStreams(uint32_t format, uint64_t groups)
+{
+  const uint64_t cus = deviceComputeUnits();
+  return format == NVPRO_PYRAMID_FORMAT_SRGBA8 && groups > cus && groups <= 64u * cus;
+}
 
 template <class F, int COUNT>
 static void launchFastCount(hipStream_t stream, const ImageDesc& img, uint32_t inLevel, uint32_t wgPerCU,
@@ -171,10 +179,8 @@ static void launchFastCount(hipStream_t stream, const ImageDesc& img, uint32_t i
     out.base[r]  = img.base + img.lv[inLevel + 1u + (uint32_t)r].offset;
     out.pitch[r] = img.lv[inLevel + 1u + (uint32_t)r].pitch;
   }
-  // Non-temporal input loads for 6-level steps in the kNtMin..kNtMaxGroupsPerCU range.
-  constexpr bool NT  = COUNT == 6;
-  const uint64_t cus = deviceComputeUnits();
-  const bool nt      = NT && groups >= kNtMinGroupsPerCU * cus && groups <= kNtMaxGroupsPerCU * cus;
+  constexpr bool NT = F::kBytes == 4u;
+  const bool nt     = fastInputStreams(img.format, groups);
   auto launch       = [&](auto kernel, auto... more) {
     hipLaunchKernelGGL(kernel, grid, wg, 0, stream, img.base + in.offset, in.pitch, tilesX * tilesY, inverse,
                        (uint16_t)tilesX, (uint16_t)blocks, more...);

@@ -205,24 +205,28 @@ static bool consecutive(const NvproPyramidStep* steps, uint32_t first, uint32_t 
   return true;
 }
 
-// Persistent workgroups per compute unit of a fast step of `groups` groups
-// (measured on MI355X, sRGBA8 F(0,6), per-step time): up to 16 groups per
-// compute unit, 8 (the most that fit: 4096^2 22.3 us; with 4 or 3, 22.6-22.8);
-// fewer workgroups on larger steps, although each then has fewer waves to
-// hide latency behind: 5120^2 (25 groups per unit) 33.2 -> 32.6 us with 4,
-// 6144^2 (36) 47.1 -> 45.2 with 3 (44.8 with 4), 8192x4096 (32) 43.0 -> 39.8 with 3, 8192^2
-// (64) 86.8 -> 76.7 with 3, 16384^2 (256) 350.1 -> 296.0 with 3 (with 2:
-// 344.3).
-static uint32_t fastWorkgroupsPerCU(uint64_t groups)
+// Persistent workgroups per compute unit of a fast step (at most 8 fit):
+// fewer than fit leave fewer waves to hide latency behind, but the rows that
+// are read at one time, which lie far apart in a large image, are fewer too.
+// Measured on MI355X, us per chain over images that are not in any cache:
+// sRGBA8 with the input loads of fastInputStreams, 5 against 8 and 4: 4096^2
+// (16 groups per unit) 22.7, 23.0, 23.4; 5120^2 34.1, 35.2, 34.0; 6144^2 45.2,
+// 44.7, 43.8; 8192^2 (64) 73.8, 75.5, 74.5; without them, 4 against 8:
+// 10240^2 123 and 132, 16384^2 (256) 323 and 345 (with 2: 350; with 3, 298 to
+// 307 against 4's 298 to 323 by where the images lie in memory).  Texels of 8
+// and 16 bytes, 2 against 8: RGBA16F 3072^2 24.9 and 27.0, 4096^2 37.9 and
+// 38.7, 12288x8192 209 and 220; RGBA32F 4096^2 69.3 and 71.4.
+static uint32_t fastWorkgroupsPerCU(const ImageDesc& img, uint64_t groups)
 {
-  const uint64_t cus = deviceComputeUnits();
-  return groups >= 32u * cus ? 3u : groups > 16u * cus ? 4u : 8u;
+  if(img.format != NVPRO_PYRAMID_FORMAT_SRGBA8)
+    return 2u;
+  return fastInputStreams(img.format, groups) || groups <= deviceComputeUnits() ? 5u : 4u;
 }
 
 static uint32_t fastWorkgroupsPerCU(const ImageDesc& img, const NvproPyramidStep& s)
 {
   const LevelDesc& in = img.lv[s.inputLevel];
-  return fastWorkgroupsPerCU(fastGroupCount(in.width, in.height, s.levelCount));
+  return fastWorkgroupsPerCU(img, fastGroupCount(in.width, in.height, s.levelCount));
 }
 
 // Whether fusing a successor into fast step s pays, by the step's workgroups
@@ -237,7 +241,7 @@ static bool fusionPays(const ImageDesc& img, const NvproPyramidStep& s)
 {
   const LevelDesc& in   = img.lv[s.inputLevel];
   const uint64_t groups = fastGroupCount(in.width, in.height, s.levelCount);
-  const uint64_t cap    = (uint64_t)fastWorkgroupsPerCU(groups) * deviceComputeUnits();
+  const uint64_t cap    = (uint64_t)fastWorkgroupsPerCU(img, groups) * deviceComputeUnits();
   const uint64_t blocks = groups < cap ? groups : cap;
   return blocks <= kArriveLeaves || blocks >= 4ull * deviceComputeUnits();
 }

@@ -126,6 +126,8 @@ constexpr uint32_t kFastTailTexels = 128;
 // plan of a kNextTail).
 hipError_t launchFast(hipStream_t stream, const ImageDesc& img, uint32_t inputLevel, uint32_t levelCount,
                       uint32_t wavesPerCU, const NextStep* next = nullptr, const TailPlan* tail = nullptr);
+// Whether a fast step of that many groups streams its input (fast_pipeline.hip).
+bool fastInputStreams(uint32_t format, uint64_t groups);
 hipError_t launchGeneral(hipStream_t stream, const ImageDesc& img, uint32_t inputLevel, uint32_t levelCount);
 hipError_t launchTail(hipStream_t stream, const ImageDesc& img, const TailPlan& plan);
 // The same steps in one launch of tiles (at most kTileSide x kTileSide texels of
