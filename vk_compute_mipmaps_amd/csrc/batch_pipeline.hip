@@ -10,8 +10,8 @@
 // loads and the general ones' plain loads with exactly the values their
 // per-step kernels see.
 //
-// Queue mode: workgroups are persistent and take the next item from an atomic
-// head counter.  Before an item of step s a workgroup waits for the completion
+// Queue mode: workgroups are persistent and take the next item (or run of items,
+// done in order) from an atomic head counter.  Before an item of step s a workgroup waits for the completion
 // counter of step s-1 to reach its item count (then drops stale cache lines);
 // an item stores its step's last level with write-through stores, waits for
 // them to complete and bumps the step's counter.  Items are taken in list
@@ -84,8 +84,13 @@ __device__ __forceinline__ void runItem(BatchShared<F>& sh, const ImageDesc* __r
   }
 }
 
+// Waves per SIMD that registers are kept for: 5 (96 registers) for sRGBA8, whose
+// bodies wait on table lookups (512 mixed images 796 us, with 4 workgroups per
+// compute unit 838); 4 (128 registers) for wider texels, whose windows take two
+// and four times the registers (128 mixed RGBA16F images 409 -> 393 us, packed
+// 403 -> 396).
 template <class F>
-__global__ void __launch_bounds__(kGroupBS) __attribute__((amdgpu_waves_per_eu(F::kBytes > 8u ? 4 : 5, 8)))
+__global__ void __launch_bounds__(kGroupBS) __attribute__((amdgpu_waves_per_eu(F::kBytes > 4u ? 4 : 5, 8)))
 batchRoundKernel(NVPRO_BATCH_PARAMS)
 {
   __shared__ BatchShared<F> sh;
@@ -101,8 +106,16 @@ batchRoundKernel(NVPRO_BATCH_PARAMS)
   }
 }
 
+// Items a workgroup takes at a time: 2 of 16-byte texels, whose items of 64 KiB
+// are a single group, so that taking them (about 14 ns each at the one head
+// word, 27075 items) bounded the launch; as long as there are this many for
+// each workgroup (64 mixed RGBA32F images: 481 -> 411 us).  Narrower texels have
+// more work in an item and lose by running ahead of their order (512 mixed
+// sRGBA8 images 796 -> 809 us with 2, 855 with 4).
+constexpr uint32_t kRunMinItems = 8;
+
 template <class F>
-__global__ void __launch_bounds__(kGroupBS) __attribute__((amdgpu_waves_per_eu(F::kBytes > 8u ? 4 : 5, 8)))
+__global__ void __launch_bounds__(kGroupBS) __attribute__((amdgpu_waves_per_eu(F::kBytes > 4u ? 4 : 5, 8)))
 batchQueueKernel(NVPRO_BATCH_PARAMS)
 {
   __shared__ BatchShared<F> sh;
@@ -111,11 +124,13 @@ batchQueueKernel(NVPRO_BATCH_PARAMS)
   uint32_t* error = counters + kCounterError;
   uint32_t* slots = counters + kCounterSlots;
   F::template fillDual<kGroupBS>(sh.tab);
+  const uint32_t run = F::kBytes > 8u && (itemEnd - itemBegin) / gridDim.x >= kRunMinItems ? 2u : 1u;
   if(threadIdx.x == 0)
-    sNext = itemBegin + __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    sNext = itemBegin + run * __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
   uint32_t iter = 0;
   uint32_t it   = __builtin_amdgcn_readfirstlane(sNext);
+  uint32_t left = run;  // items of the run from `it` on
   while(it < itemEnd)
   {
     const QueueItem item = items[it];
@@ -123,10 +138,11 @@ batchQueueKernel(NVPRO_BATCH_PARAMS)
     uint32_t next        = 0;
     if(threadIdx.x == 0)
     {
-      // Take the next item now so its latency overlaps this one.  Items are taken
-      // in order and this one is finished before the next starts, so holding it
+      // Take the next run now so its latency overlaps this item.  Runs are taken
+      // in order and this item is finished before the next starts, so holding it
       // early cannot block anything.
-      next = itemBegin + __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if(left == 1u)
+        next = itemBegin + run * __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if(seg.depSlot != kNoSlot)
         waitCounter(slots + seg.depSlot, seg.depCount, spinLimit, error);
     }
@@ -147,10 +163,11 @@ batchQueueKernel(NVPRO_BATCH_PARAMS)
     {
       if(seg.doneSlot != kNoSlot)
         __hip_atomic_fetch_add(slots + seg.doneSlot, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      sNext = next;
+      sNext = left == 1u ? next : it + 1u;
     }
     __syncthreads();
-    it = __builtin_amdgcn_readfirstlane(sNext);
+    it   = __builtin_amdgcn_readfirstlane(sNext);
+    left = left == 1u ? run : left - 1u;
   }
   // Exit: the last workgroup out resets the counters for the next launch.  Every
   // other workgroup has made its last head and slot update by then.
