@@ -274,7 +274,7 @@ def main():
         "chain_roofline_frac": round(chain_total_bytes / (us_per_chain * 1e-6) / 1e9 / HBM_PEAK_GBS, 4),
         "roofline": {
             "bound": "hbm",
-            "kernel": "fastPipelineKernel<Srgba8, 6, true> (the chain's one launch: F(0,6), then F(6,6) "
+            "kernel": "fastFusedKernel<Srgba8, 6, true> (the chain's one launch: F(0,6), then F(6,6) "
                       "in its last workgroup)",
             "achieved": round(chain_total_bytes / (us_per_chain * 1e-6) / 1e9, 1),
             "peak": HBM_PEAK_GBS,
@@ -286,7 +286,7 @@ def main():
             "timing": "HIP events on the dispatch stream over the timed region; one launch per chain",
         },
         "first_step_alone": {
-            "kernel": "fastPipelineKernel<Srgba8, 6, false> (F(0,6) over level 0, mipLevels 7)",
+            "kernel": "fastPipelineKernel<Srgba8, 6, true> (F(0,6) over level 0, mipLevels 7)",
             "us": round(k_us, 3),
             "GBps": round(k_gbs, 1),
             "frac": round(k_gbs / HBM_PEAK_GBS, 4),

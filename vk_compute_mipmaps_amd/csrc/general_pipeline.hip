@@ -86,23 +86,30 @@ static uint32_t residentPerCU(K kernel, int threads)
   return (uint32_t)n;
 }
 
-// A step whose thin tiles all fit on the GPU at once runs them: its time is then
-// one tile's latency, and a thin tile's lanes run less serial work than a
-// strip's.  A larger one runs strips.  A step with a first-level side of 1 always runs
+// A step with at most two thin tiles per compute unit runs thin tiles: its time
+// is then one tile's latency, and a thin tile's lanes run less serial work than
+// a strip's.  A larger one runs strips, which decode and load less at the
+// borders (us per G(0,2), thin and strips; sRGBA8: 801x401, 238 thin tiles, 4.4
+// and 4.6; 1001x501, 378 tiles, 4.9 and 4.6, but after a larger step, whose
+// output is in the caches, thin: 2047x1023 chains 18.7 and 19.5; 1201x701, 590 tiles, 5.5 and 4.9; 2002x1234
+// 8.05 and 6.5; RGBA16F 4.3 and 4.4, 4.8 and 4.4, 5.6 and 4.9, 9.1 and 8.4).
+// 16-byte texels run thin tiles while they all fit on the GPU at once (RGBA32F
+// 1001x501 5.7 and 6.5, 2002x1234 14.3 and 15.4; in between, 1501x1001, 10.3 and
+// 8.9).  A step with a first-level side of 1 always runs
 // thin tiles (a 65535-texel side has 529 of them).  The environment variable
 // NVPRO_PYRAMID_THIN=1 / =0 forces thin tiles / strips where both apply (the
 // bytes are the same either way).
 template <class F, int KX, int KY>
 static void launchTwoLevel(hipStream_t stream, const ImageDesc& img, uint32_t inLevel)
 {
-  static const uint32_t fitThin = residentPerCU(thinTwoLevelKernel<F, KX, KY>, kGroupBS);
-  const LevelDesc& d            = img.lv[inLevel + 2u];
-  uint32_t thinX                = 0;
+  static const uint32_t perCU = F::kBytes > 8u ? residentPerCU(thinTwoLevelKernel<F, KX, KY>, kGroupBS) : 2u;
+  const LevelDesc& d          = img.lv[inLevel + 2u];
+  uint32_t thinX              = 0;
   const uint32_t numThin = generalGroupCount(d.width, d.height, 2u, F::kBytes, &thinX, true);
   const char* force      = getenv("NVPRO_PYRAMID_THIN");
   const bool thin        = force && (force[0] == '0' || force[0] == '1')
                                ? force[0] == '1'
-                               : (uint64_t)numThin <= (uint64_t)deviceComputeUnits() * fitThin;
+                               : (uint64_t)numThin <= (uint64_t)deviceComputeUnits() * perCU;
   if constexpr(KX != 0 && KY != 0)
     if(!thin && stripsApply(img, inLevel))
     {
