@@ -243,7 +243,7 @@ static uint32_t fastWorkgroupsPerCU(const ImageDesc& img, const NvproPyramidStep
 // kernel, the write-back of everything it stored (2048 workgroups of 4096^2
 // with F(6,6): 28.1 -> 26.5 us per chain); in between, two arrival counts and
 // the continuation cost what they save (256 workgroups of 1024^2 with F(6,4):
-// 8.7 -> 9.2 us).
+// 7.4 -> 8.2 us).
 static bool fusionPays(const ImageDesc& img, const NvproPyramidStep& s)
 {
   const LevelDesc& in   = img.lv[s.inputLevel];
