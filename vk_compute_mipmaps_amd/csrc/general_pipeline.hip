@@ -27,6 +27,8 @@ __global__ void __launch_bounds__(kGroupBS) generalOneLevelKernel(ImageDesc img,
 }
 
 // Thin tiles, one per workgroup (the grid is numTiles): straight-line code.
+// The window's loads are issued behind the tables', one memory round trip for
+// both (2002x1234 RGBA32F chain 23.6 -> 23.2 us, 801x401 sRGBA8 14.7 -> 14.1).
 // KX, KY: the first level's kernel sizes, or 0 (read from the image).
 template <class F, int KX, int KY>
 __global__ void __launch_bounds__(kGroupBS) thinTwoLevelKernel(ImageDesc img, uint32_t inLevel, uint32_t tilesX,
@@ -35,11 +37,15 @@ __global__ void __launch_bounds__(kGroupBS) thinTwoLevelKernel(ImageDesc img, ui
   __shared__ ThinShared<F> sh;
   if(blockIdx.x >= numTiles)  // the same for the whole workgroup
     return;
+  typename F::template TableLoads<kGroupBS> tables;
+  F::template fillLoad<kGroupBS>(tables);
   const uint32_t lines = prefetchLevels(img);
-  F::template fill<kGroupBS>(sh.tab, 1.0f);
+  Gen2Window<F, true> w;
+  gen2Load<F, KX, KY, true>(img, inLevel, tilesX, blockIdx.x, w);
+  F::template fillStore<kGroupBS>(sh.tab, tables, 1.0f);
   __syncthreads();
   levelsReady(lines);
-  generalTwoGroup<F, false, KX, KY, true>(sh.tab, sh.mid, img, inLevel, tilesX, blockIdx.x);
+  gen2Compute<F, false, KX, KY, true>(sh.tab, sh.mid, img, inLevel, tilesX, blockIdx.x, w);
 }
 
 // One strip group per workgroup, strips of a row of groups side by side, in the
