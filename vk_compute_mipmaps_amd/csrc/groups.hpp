@@ -299,11 +299,9 @@ __device__ __forceinline__ void fastCompute(const TT& tab, typename F::Val* leve
 
 // Group g, loads included.  Contains barriers when COUNT >= 3.  CO: the last
 // level is stored with storeTexelCoherent (for a continuation in the same
-// launch, see arriveLast).  STRIP: the lane layout (fastLanePos).  NT: the
-// input loads carry the non-temporal hint.  HOIST: output addressing read up
-// front (FastOut).
-template <class F, int COUNT, bool CO = false, bool STRIP = (COUNT == 6), bool NT = false, bool HOIST = true,
-          class TT>
+// launch, see arriveLast).  STRIP: the lane layout (fastLanePos).  HOIST: output
+// addressing read up front (FastOut).
+template <class F, int COUNT, bool CO = false, bool STRIP = (COUNT == 6), bool HOIST = true, class TT>
 __device__ __forceinline__ void fastGroup(const TT& tab, typename F::Val* level2, const ImageDesc& img,
                                           uint32_t inLevel, uint32_t tilesX, uint32_t numTiles, uint32_t g,
                                           uint32_t iter)
@@ -312,7 +310,7 @@ __device__ __forceinline__ void fastGroup(const TT& tab, typename F::Val* level2
   const FastTiles tiles{tilesX, numTiles};
   const FastOut<COUNT, HOIST> out(img, inLevel);
   FastWindow<F, COUNT> w;
-  fastLoad<F, COUNT, STRIP, NT>(img.base + in.offset, in.pitch, tiles, g, threadIdx.x, w);
+  fastLoad<F, COUNT, STRIP, false>(img.base + in.offset, in.pitch, tiles, g, threadIdx.x, w);
   fastCompute<F, COUNT, CO, STRIP>(tab, level2, out, tiles, g, iter, threadIdx.x, w);
 }
 
@@ -615,14 +613,14 @@ __device__ __forceinline__ void gen2Compute(const TT& tab, typename F::Val* mid,
   __syncthreads();
 }
 
-// One tile.  Contains barriers.
-template <class F, bool CO = false, int KX = 0, int KY = 0, bool THIN = false, class TT>
+// One full tile, loads included.  Contains barriers.
+template <class F, bool CO = false, int KX = 0, int KY = 0, class TT>
 __device__ __forceinline__ void generalTwoGroup(const TT& tab, typename F::Val* mid, const ImageDesc& img,
                                                 uint32_t inLevel, uint32_t tilesX, uint32_t tile)
 {
-  Gen2Window<F, THIN> w;
-  gen2Load<F, KX, KY, THIN>(img, inLevel, tilesX, tile, w);
-  gen2Compute<F, CO, KX, KY, THIN>(tab, mid, img, inLevel, tilesX, tile, w);
+  Gen2Window<F> w;
+  gen2Load<F, KX, KY>(img, inLevel, tilesX, tile, w);
+  gen2Compute<F, CO, KX, KY>(tab, mid, img, inLevel, tilesX, tile, w);
 }
 
 // One tile, through the specialisation for the first level's kernel sizes
