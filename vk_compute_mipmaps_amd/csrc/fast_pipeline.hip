@@ -110,7 +110,7 @@ fastPipelineKernel(const uint8_t* src, uint32_t pitch, uint32_t numTiles, uint32
                    uint16_t blocks, FastOut<COUNT, true> out)
 {
   __shared__ FastShared<F, COUNT, false> sh;
-  fastGroups<F, COUNT, false, NT>(sh, src, pitch, FastTilesInverse{tilesX, numTiles, tilesInverse}, blocks, out, 0u);
+  fastGroups<F, COUNT, false, NT>(sh, src, pitch, FastTilesInverse(tilesX, numTiles, tilesInverse), blocks, out, 0u);
 }
 
 // The same and then, in the last workgroup, the successor (a NextStep's fields).
@@ -122,7 +122,7 @@ fastFusedKernel(const uint8_t* src, uint32_t pitch, uint32_t numTiles, uint32_t 
 {
   __shared__ FastShared<F, COUNT, true> sh;
   const uint32_t lines = prefetchLevels(img);
-  const FastTilesInverse tiles{tilesX, numTiles, tilesInverse};
+  const FastTilesInverse tiles(tilesX, numTiles, tilesInverse);
   const uint32_t iter = fastGroups<F, COUNT, true, NT>(sh, src, pitch, tiles, blocks, out, lines);
   if(!arriveLast(arrive, blocks, reinterpret_cast<uint32_t*>(sh.level2)))
     return;
@@ -172,7 +172,7 @@ static void launchFastCount(hipStream_t stream, const ImageDesc& img, uint32_t i
   const uint64_t cap      = min((uint64_t)deviceComputeUnits() * wgPerCU, (uint64_t)0xffffu);
   const uint32_t blocks   = (uint32_t)(groups < cap ? groups : cap);
   const dim3 grid(blocks), wg(kGroupBS);
-  const uint32_t inverse = (uint32_t)((0x100000000ull + tilesX - 1u) / tilesX);
+  const uint32_t inverse  = FastTilesInverse::inverseOf(tilesX);
   FastOut<COUNT, true> out;
   for(int r = 0; r < COUNT; ++r)
   {

@@ -87,18 +87,37 @@ __host__ __device__ inline uint32_t fastGroupCount(uint32_t width, uint32_t heig
   return (tiles + perWG - 1u) / perWG;
 }
 
-// The tiles of a fast step: `x` in a row, `count` in all; row(tile) is
-// tile / x, by multiplication where the host prepared the inverse (2^32 / x,
-// rounded up: exact while tile * x < 2^32).
+// The tiles of a fast step: `x` in a row, `count` in all; row(tile) is tile / x.
 struct FastTiles
 {
   uint32_t x, count;
   __device__ __forceinline__ uint32_t row(uint32_t tile) const { return tile / x; }
 };
+// The same by multiplication with an inverse made on the host: with `shift` the
+// number for which 2^shift < x <= 2^(shift + 1), inverse = 2^(32 + shift) / x
+// rounded up, which fits 32 bits.  inverse * x is then above 2^(32 + shift) by
+// e < x, and the quotient is exact while tile * e < 2^(32 + shift): for every
+// tile below 2^31, whatever x (a level's sides are below 65536, so a step has
+// fewer than 2^30 tiles).
 struct FastTilesInverse
 {
-  uint32_t x, count, inverse;
-  __device__ __forceinline__ uint32_t row(uint32_t tile) const { return x == 1u ? tile : __umulhi(tile, inverse); }
+  uint32_t x, count, inverse, shift;
+  __host__ __device__ __forceinline__ static uint32_t shiftOf(uint32_t x)
+  {
+    return x > 1u ? 31u - (uint32_t)__builtin_clz(x - 1u) : 0u;
+  }
+  __host__ static uint32_t inverseOf(uint32_t x)
+  {
+    return x > 1u ? (uint32_t)(((0x100000000ull << shiftOf(x)) + x - 1u) / x) : 0u;
+  }
+  __host__ __device__ __forceinline__ FastTilesInverse(uint32_t x_, uint32_t count_, uint32_t inverse_)
+      : x(x_), count(count_), inverse(inverse_), shift(shiftOf(x_))
+  {
+  }
+  __host__ __device__ __forceinline__ uint32_t row(uint32_t tile) const
+  {
+    return x == 1u ? tile : (uint32_t)((uint64_t)tile * inverse >> 32) >> shift;
+  }
 };
 
 // The input block of one lane for group g of a fast step: its 2^LB rows, all
