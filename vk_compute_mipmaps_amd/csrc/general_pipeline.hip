@@ -277,10 +277,13 @@ hipError_t executePlan(hipStream_t stream, const ImageDesc& img, const NvproPyra
     if(arrive && i + 1u < count && fast && fusionPays(img, s))
     {
       // Fusion: the successor runs in this launch's last workgroup, saving a
-      // launch and the second kernel's start-up (tables, first loads).
+      // launch and the second kernel's start-up (tables, first loads).  It has to
+      // read this step's last level, the only one stored for other workgroups to
+      // see, and a tail's steps each the one before's.
       const NvproPyramidStep& n = steps[i + 1u];
       const LevelDesc& nin      = img.lv[n.inputLevel];
-      if(n.pipeline == NVPRO_PYRAMID_PIPELINE_FAST && fastGroupCount(nin.width, nin.height, n.levelCount) == 1u)
+      if(n.pipeline == NVPRO_PYRAMID_PIPELINE_FAST && fastGroupCount(nin.width, nin.height, n.levelCount) == 1u
+         && consecutive(steps, i, i + 2u))
       {
         const uint32_t tilesX = nin.width >> n.levelCount, tilesY = nin.height >> n.levelCount;
         const NextStep next{arrive, kNextFast, n.inputLevel, n.levelCount, tilesX, tilesX * tilesY};
@@ -293,7 +296,7 @@ hipError_t executePlan(hipStream_t stream, const ImageDesc& img, const NvproPyra
       // followed by a tail measured no faster fused: the tail's first level
       // then takes several passes of a 256-thread workgroup, where the tail
       // kernel takes one pass of 1024 threads.)
-      if(firstOutput(img, n) <= kFastTailTexels)
+      if(firstOutput(img, n) <= kFastTailTexels && consecutive(steps, i, count))
       {
         const TailPlan tail = tailFrom(steps, i + 1u, count);
         const NextStep next{arrive, kNextTail, 0u, 0u, 0u, 0u};
