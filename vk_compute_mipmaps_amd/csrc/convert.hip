@@ -9,7 +9,7 @@
 //
 // A byte in and a byte out per byte of the level: bound by memory once a thread
 // moves four texels an access.  Workgroups take segments of a row, so that the
-// only division is one of scalars per segment.  (A thread per texel with a
+// only division is one of scalars per segment (narrow rows with padding: below).  (A thread per texel with a
 // 64-bit division each was bound by those: 3840x2160 sRGBA8, level 0 in the
 // caches, 18.3 us; now 13.7.  One access in flight a thread 14.1, four 13.9.)
 #include "kernel_common.hpp"
@@ -81,6 +81,74 @@ __global__ void __launch_bounds__(kPremultiplyBS) premultiplyKernel(uint8_t* bas
   }
 }
 
+// Narrow rows longer than the level: a segment's workgroup has little to do in a
+// row of them, so here a workgroup takes units of `rows` rows, as many as there
+// are whole ones in kNarrowAhead texels a thread, a texel per lane and access,
+// all loads of a unit in flight at once.  A texel's row in the unit is
+// t / width = t * inverse >> 20, exact while t * width < 2^20.  (Level 0 in the
+// caches, us a call with a segment a row and with units: sRGBA8 64x16384 10.1 and
+// 4.0, 16x65535 32.8 and 4.0, 300x9000 8.6 and 5.7, RGBA16F 64x16384 9.2 and 3.9;
+// calls this small come every 4 us at best.  Wider rows fill their segments better
+// and would leave more of a unit idle: 700x5000 7.6 with segments, and a thread
+// per texel with a division each, 9.4.)
+constexpr uint32_t kNarrowMost = 512, kNarrowAhead = 8;
+static_assert(kNarrowAhead * kPremultiplyBS * kNarrowMost <= 1u << 20, "exact rows");
+
+template <class P>
+__global__ void __launch_bounds__(kPremultiplyBS) premultiplyNarrowKernel(uint8_t* base, uint32_t width, uint32_t height,
+                                                                         uint32_t pitch, uint32_t inverse,
+                                                                         uint32_t rows, uint32_t units)
+{
+  __shared__ typename P::Tables tab;
+  P::template fill<kPremultiplyBS>(tab, 1.0f);
+  __syncthreads();
+  for(uint32_t u = blockIdx.x; u < units; u += gridDim.x)
+  {
+    const uint32_t first = u * rows;
+    const uint32_t count = height - first < rows ? height - first : rows;
+    uint8_t* p[kNarrowAhead];
+    bool own[kNarrowAhead];
+    typename P::Raw t[kNarrowAhead];
+#pragma unroll
+    for(uint32_t a = 0; a < kNarrowAhead; ++a)
+    {
+      // No branch around the loads: past the unit its last row's texels, unused.
+      const uint32_t i = a * kPremultiplyBS + threadIdx.x, r = __umul24(i, inverse) >> 20;
+      own[a] = r < count;
+      p[a]   = base + (uint64_t)(first + (own[a] ? r : count - 1u)) * pitch + (i - __umul24(r, width)) * P::kBytes;
+      t[a] = loadTexel<P>(p[a]);
+    }
+#pragma unroll
+    for(uint32_t a = 0; a < kNarrowAhead; ++a)
+      if(own[a])
+        storeTexel<P>(p[a], P::texel(tab, t[a]));
+  }
+}
+
+template <class P>
+static void launchPremultiply(hipStream_t stream, uint8_t* base, uint32_t imageWidth, uint32_t imageHeight, uint32_t pitch)
+{
+  // Rows without padding are one long row.
+  const bool tight   = pitch == (uint64_t)imageWidth * P::kBytes;
+  const uint64_t cap = deviceComputeUnits() * 8u;
+  if(!tight && imageWidth <= kNarrowMost)
+  {
+    const uint32_t rows    = kNarrowAhead * kPremultiplyBS / imageWidth;
+    const uint32_t units   = imageHeight / rows + (imageHeight % rows ? 1u : 0u);
+    const uint32_t inverse = ((1u << 20) + imageWidth - 1u) / imageWidth;
+    const uint32_t grid    = (uint32_t)(units < cap ? units : cap);
+    hipLaunchKernelGGL((premultiplyNarrowKernel<P>), dim3(grid), dim3(kPremultiplyBS), 0, stream, base, imageWidth,
+                       imageHeight, pitch, inverse, rows, units);
+    return;
+  }
+  const uint64_t width    = (uint64_t)imageWidth * (tight ? imageHeight : 1u);
+  const uint64_t segments = (width + kPremultiplySegment - 1u) / kPremultiplySegment;
+  const uint64_t units    = segments * (tight ? 1u : imageHeight);
+  const uint32_t grid     = (uint32_t)(units < cap ? units : cap);
+  hipLaunchKernelGGL((premultiplyKernel<P>), dim3(grid), dim3(kPremultiplyBS), 0, stream, base, width, pitch, segments,
+                     units);
+}
+
 }  // namespace nvpro_pyramid
 
 using namespace nvpro_pyramid;
@@ -100,20 +168,11 @@ extern "C" int nvproPyramidPremultiplyAlpha(hipStream_t stream, uint32_t format,
   if(pitch < (uint64_t)image->width * bpt || pitch > 0xffffffffull || pitch % bpt != 0 ||
      (((uintptr_t)image->data + off) % bpt) != 0)
     return hostFail(hipErrorInvalidValue, "%s: level 0 layout not aligned to %u bytes", who, bpt);
-  uint8_t* base       = (uint8_t*)image->data + off;
-  // Rows without padding are one long row.
-  const bool tight        = pitch == (uint64_t)image->width * bpt;
-  const uint64_t width    = (uint64_t)image->width * (tight ? image->height : 1u);
-  const uint64_t segments = (width + kPremultiplySegment - 1u) / kPremultiplySegment;
-  const uint64_t units    = segments * (tight ? 1u : image->height);
-  const uint64_t cap  = deviceComputeUnits() * 8u;
-  const uint32_t grid = (uint32_t)(units < cap ? units : cap);
+  uint8_t* base = (uint8_t*)image->data + off;
   if(format == NVPRO_PYRAMID_FORMAT_SRGBA8)
-    hipLaunchKernelGGL((premultiplyKernel<PremultiplySrgba8>), dim3(grid), dim3(kPremultiplyBS), 0, stream, base,
-                       width, (uint32_t)pitch, segments, units);
+    launchPremultiply<PremultiplySrgba8>(stream, base, image->width, image->height, (uint32_t)pitch);
   else
-    hipLaunchKernelGGL((premultiplyKernel<PremultiplyRgba16f>), dim3(grid), dim3(kPremultiplyBS), 0, stream, base,
-                       width, (uint32_t)pitch, segments, units);
+    launchPremultiply<PremultiplyRgba16f>(stream, base, image->width, image->height, (uint32_t)pitch);
   hipError_t e = hipGetLastError();
   if(e != hipSuccess)
     return hostFail(e, "%s: launch failed: %s", who, hipGetErrorString(e));
