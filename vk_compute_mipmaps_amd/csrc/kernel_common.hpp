@@ -75,14 +75,15 @@ __device__ __forceinline__ void loadRow(const uint8_t* p, typename F::Raw (&out)
 }
 
 // loadRow for data read once: 16-byte loads with the non-temporal hint (rows
-// whose size is not a multiple of 16 bytes load as loadRow does).
+// whose size is not a multiple of 16 bytes load as loadRow does).  The vector's
+// alignment is what a row has, 4 bytes.
 template <class F, int N>
 __device__ __forceinline__ void loadRowStream(const uint8_t* p, typename F::Raw (&out)[N])
 {
   constexpr int NBYTES = N * F::kBytes;
   if constexpr(NBYTES % 16 == 0)
   {
-    typedef uint32_t U4 __attribute__((ext_vector_type(4)));
+    typedef uint32_t U4 __attribute__((ext_vector_type(4), aligned(4)));
     uint32_t w[NBYTES / 4];
 #pragma unroll
     for(int i = 0; i < NBYTES / 16; ++i)
