@@ -65,7 +65,7 @@ static_assert(2u * kFastTailTexels <= (uint32_t)kGroupBS, "tail ping-pong fits t
 // Returns how many groups it ran.
 template <class F, int COUNT, bool CONT, bool NT>
 __device__ __forceinline__ uint32_t fastGroups(FastShared<F, COUNT, CONT>& sh, const uint8_t* src, uint32_t pitch,
-                                               const FastTilesInverse& tiles, uint32_t blocks,
+                                               const FastTilesInverse<COUNT>& tiles, uint32_t blocks,
                                                const FastOut<COUNT, true>& out, uint32_t lines)
 {
   constexpr bool STRIP     = COUNT == 6;
@@ -110,7 +110,7 @@ fastPipelineKernel(const uint8_t* src, uint32_t pitch, uint32_t numTiles, uint32
                    uint16_t blocks, FastOut<COUNT, true> out)
 {
   __shared__ FastShared<F, COUNT, false> sh;
-  fastGroups<F, COUNT, false, NT>(sh, src, pitch, FastTilesInverse(tilesX, numTiles, tilesInverse), blocks, out, 0u);
+  fastGroups<F, COUNT, false, NT>(sh, src, pitch, FastTilesInverse<COUNT>(tilesX, numTiles, tilesInverse), blocks, out, 0u);
 }
 
 // The same and then, in the last workgroup, the successor (a NextStep's fields).
@@ -122,7 +122,7 @@ fastFusedKernel(const uint8_t* src, uint32_t pitch, uint32_t numTiles, uint32_t 
 {
   __shared__ FastShared<F, COUNT, true> sh;
   const uint32_t lines = prefetchLevels(img);
-  const FastTilesInverse tiles(tilesX, numTiles, tilesInverse);
+  const FastTilesInverse<COUNT> tiles(tilesX, numTiles, tilesInverse);
   const uint32_t iter = fastGroups<F, COUNT, true, NT>(sh, src, pitch, tiles, blocks, out, lines);
   if(!arriveLast(arrive, blocks, reinterpret_cast<uint32_t*>(sh.level2)))
     return;
@@ -172,7 +172,7 @@ static void launchFastCount(hipStream_t stream, const ImageDesc& img, uint32_t i
   const uint64_t cap      = min((uint64_t)deviceComputeUnits() * wgPerCU, (uint64_t)0xffffu);
   const uint32_t blocks   = (uint32_t)(groups < cap ? groups : cap);
   const dim3 grid(blocks), wg(kGroupBS);
-  const uint32_t inverse  = FastTilesInverse::inverseOf(tilesX);
+  const uint32_t inverse  = FastTilesInverse<COUNT>::inverseOf(tilesX);
   FastOut<COUNT, true> out;
   for(int r = 0; r < COUNT; ++r)
   {
