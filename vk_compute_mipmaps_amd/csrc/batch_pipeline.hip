@@ -77,7 +77,7 @@ __device__ __forceinline__ void runItem(BatchShared<F>& sh, const ImageDesc* __r
       case kSegGeneral1: generalOneGroup<F, CO>(sh.tab, img, seg.inputLevel, g); break;
       case kSegGeneral2: generalTwoGroupAny<F, CO>(sh.tab, scratch, img, seg.inputLevel, seg.tilesX, g); break;
       case kSegTail:
-        tailRun<F, kGroupBS>(sh.tab, scratch, scratch + kBatchTailTexels, img, tails[seg.inputLevel]);
+        tailRun<F>(sh.tab, scratch, scratch + kBatchTailTexels, img, tails[seg.inputLevel]);
         break;
       default: break;
     }

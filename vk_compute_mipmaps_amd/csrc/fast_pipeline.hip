@@ -133,7 +133,7 @@ fastFusedKernel(const uint8_t* src, uint32_t pitch, uint32_t numTiles, uint32_t 
       F::template fill<kGroupBS>(sh.tab, 1.0f);
       __syncthreads();
     }
-    tailRun<F, kGroupBS, 1, false>(sh.tab, sh.level2, sh.level2 + kFastTailTexels, img, tail);
+    tailRun<F, false>(sh.tab, sh.level2, sh.level2 + kFastTailTexels, img, tail);
     return;
   }
   switch(nextCount)

@@ -99,9 +99,9 @@ struct FastTiles
 // 65536, so six-level steps have x < 2^10 and fewer than 2^20 tiles: exact with
 // shift = 0.  The others take the shift for which 2^shift < x <= 2^(shift + 1),
 // the largest that keeps the inverse in 32 bits: exact for every tile below
-// 2^31 whatever x is, and they have fewer than 2^30.  (The shift is found from x:
-// with it 256^2 chains, of six-level steps, take 6.33 us,
-// without it 6.26.)
+// 2^31 whatever x is, and they have fewer than 2^30.  (Finding the
+// shift costs a launch's start: 256^2 chains of six-level steps 6.33 us with it,
+// 6.26 without.)
 template <int COUNT>
 struct FastTilesInverse
 {
@@ -997,7 +997,7 @@ __device__ __forceinline__ void stripCompute(const TT& tab, typename F::Val* bor
 // that of the per-step bodies (fast: box with the reference's order; general:
 // reduceStoreSample_), so results do not depend on which kernel ran a step.
 // `buf0`, `buf1`: LDS ping-pong of maxTexels values each, where maxTexels is at
-// least the first output level's texel count.  BS threads (the workgroup).
+// least the first output level's texel count.  kGroupBS threads (the workgroup).
 // Contains barriers.
 // ---------------------------------------------------------------------------
 
@@ -1023,12 +1023,10 @@ __device__ __forceinline__ void tailLoad(const ImageDesc& img, const LevelDesc& 
         w.raw[k][j] = loadTexel<F>(q + (uint64_t)k * sl.pitch + (uint64_t)j * F::kBytes);
 }
 
-// The first level reads memory: its outputs go in chunks of PF passes of the
-// workgroup, every load of a chunk issued before its arithmetic, so a chunk
-// pays one memory latency instead of one per pass (9 PF texels of registers).
+// The first level reads memory, a window's loads all issued before its arithmetic.
 // SPEC: general levels through generalSampleAny (constant kernel sizes, more
 // code); off where registers are tight.
-template <class F, int BS, int PF = 1, bool SPEC = true, class TT>
+template <class F, bool SPEC = true, class TT>
 __device__ __forceinline__ void tailRun(const TT& tab, typename F::Val* buf0, typename F::Val* buf1,
                                         const ImageDesc& img, const TailPlan& plan)
 {
@@ -1058,34 +1056,20 @@ __device__ __forceinline__ void tailRun(const TT& tab, typename F::Val* buf0, ty
       };
       if(!cur)
       {
-        for(uint32_t base = 0; base < n; base += PF * BS)
+        for(uint32_t i = threadIdx.x; i < n; i += kGroupBS)
         {
-          TailWindow<F> win[PF];
-#pragma unroll
-          for(int p = 0; p < PF; ++p)
-          {
-            const uint32_t i = base + (uint32_t)p * BS + threadIdx.x;
-            if(i < n)
-              tailLoad<F>(img, sl, dl, i, win[p]);
-          }
-#pragma unroll
-          for(int p = 0; p < PF; ++p)
-          {
-            const uint32_t i = base + (uint32_t)p * BS + threadIdx.x;
-            if(i < n)
-            {
-              const uint32_t dy = i / dl.width, dx = i - dy * dl.width;
-              auto at = [&](int j, int k) -> V { return F::template load<false>(tab, win[p].raw[k][j]); };
-              finish(i, dx, dy, fast ? box<F, false>(at(0, 0), at(1, 0), at(0, 1), at(1, 1), order)
-                                     : (SPEC ? generalSampleAny<F>(at, kx, ky, ax, ay, dx, dy)
-                                            : generalSample<F>(at, kx, ky, ax, ay, dx, dy)));
-            }
-          }
+          TailWindow<F> win;
+          tailLoad<F>(img, sl, dl, i, win);
+          const uint32_t dy = i / dl.width, dx = i - dy * dl.width;
+          auto at = [&](int j, int k) -> V { return F::template load<false>(tab, win.raw[k][j]); };
+          finish(i, dx, dy, fast ? box<F, false>(at(0, 0), at(1, 0), at(0, 1), at(1, 1), order)
+                                 : (SPEC ? generalSampleAny<F>(at, kx, ky, ax, ay, dx, dy)
+                                        : generalSample<F>(at, kx, ky, ax, ay, dx, dy)));
         }
       }
       else
       {
-        for(uint32_t i = threadIdx.x; i < n; i += BS)
+        for(uint32_t i = threadIdx.x; i < n; i += kGroupBS)
         {
           const uint32_t dy = i / dl.width, dx = i - dy * dl.width;
           auto at = [&](int j, int k) -> V { return cur[(2u * dy + (uint32_t)k) * sl.width + 2u * dx + (uint32_t)j]; };
