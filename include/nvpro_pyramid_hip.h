@@ -143,7 +143,8 @@ uint32_t nvproPyramidDefaultGeneralDispatcher(NvproPyramidCmd* cmd, const NvproP
  * texels run in one launch, and a fast step (of at most 64 or at least 1024
  * workgroups) whose successor is a fast step of one workgroup, or the rest of
  * the plan with at most 128 texels in its first output level, runs that in its
- * own launch, in whichever workgroup finishes last.  Two steps or more of at
+ * own launch, in whichever workgroup finishes last (steps share a launch only
+ * where each starts at the level the one before it ends with).  Two steps or more of at
  * most four levels together, small enough that tiles of at most 4x4 texels of
  * their last level are no more than the compute units, run in one launch too;
  * sRGBA8 steps that a general step begins do so only where the second could be

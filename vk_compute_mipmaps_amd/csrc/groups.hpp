@@ -683,9 +683,10 @@ __device__ __forceinline__ void generalTwoGroupAny(const TT& tab, typename F::Va
 // Every value is generalSample's, from the same operands in the same order.
 // Both first-level sides must be at least 2 (so the input's at least 4).
 //
-// What bounds it (MI355X, 4095^2 sRGBA8): VALU issue (411 instructions a wave
-// of 63 x 1 second-level texels, about half of the time), the LDS lookups' bank
-// conflicts and memory each come to 50-75 % of the time.  The 31 x 7 tiles it
+// What bounds it (MI355X, 4095^2 sRGBA8, 23.9 us): no one unit.  Its memory
+// accesses alone take 18 us, its VALU instructions (414 a wave of 63 x 1
+// second-level texels) 13.5 at 4 cycles each, its LDS lookups with their bank
+// conflicts 12.8; what is left is how well these overlap.  The 31 x 7 tiles it
 // replaced (a lane per first-level column, the second level from LDS) issued
 // 50 % more VALU instructions per texel and read the input in dwords: G(0,2) of
 // 4095^2 30.1 -> 25.0 us, 8191^2 105 -> 78, 4095x2047 18.4 -> 14.2, RGBA16F
