@@ -9,9 +9,10 @@
 //
 // A byte in and a byte out per byte of the level: bound by memory once a thread
 // moves four texels an access.  Workgroups take segments of a row, so that the
-// only division is one of scalars per segment (narrow rows with padding: below).  (A thread per texel with a
-// 64-bit division each was bound by those: 3840x2160 sRGBA8, level 0 in the
-// caches, 18.3 us; now 13.7.  One access in flight a thread 14.1, four 13.9.)
+// only division is one of scalars per segment; narrow rows with padding have a
+// kernel of their own, below.  (A thread per texel with a 64-bit division each
+// was bound by those: 3840x2160 sRGBA8, level 0 in the caches, 18.3 us; now 13.7.
+// One access in flight a thread 14.1, four 13.9.)
 #include "kernel_common.hpp"
 
 namespace nvpro_pyramid {
